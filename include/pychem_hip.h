@@ -361,6 +361,21 @@ int pq_mlp_mse(const float* Y, const float* T, const float* mask, float* dY, flo
                float inv_norm, void* stream);
 int pq_mlp_adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2, float eps,
                 int step, void* stream);
+/* A whole network in one launch (gradients in two): nlayer (<= 8) layers of
+ * widths dims[nlayer + 1], hidden layers tanh, the last layer linear; the
+ * arrays are host arrays of device pointers, one per layer.
+ * forward: A[l] [B x dims[l+1]] receives layer l's output; NULL for a hidden
+ * layer that is not wanted (all are needed when a width exceeds 448).
+ * backward: A[l] the hidden layers' outputs, dY the gradient of the last
+ * layer's output; dZ[l] [B x dims[l+1]] scratch of the hidden layers; dW, db
+ * receive the gradients.
+ * adam_multi: pq_mlp_adam over nt (<= 16) tensors of n[t] elements. */
+int pq_mlp_forward(int nlayer, const int* dims, const float* X, const float* const* W, const float* const* b,
+                   float* const* A, int B, void* stream);
+int pq_mlp_backward(int nlayer, const int* dims, const float* X, const float* const* A, const float* const* W,
+                    const float* dY, float* const* dZ, float* const* dW, float* const* db, int B, void* stream);
+int pq_mlp_adam_multi(int nt, float* const* p, const float* const* g, float* const* m, float* const* v,
+                      const long long* n, float lr, float b1, float b2, float eps, int step, void* stream);
 
 #ifdef __cplusplus
 }

@@ -84,6 +84,11 @@ SIGNATURES = {
     "pq_mlp_mse": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, ctypes.c_float, c_void_p]),
     "pq_mlp_adam": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, ctypes.c_float, ctypes.c_float,
                             ctypes.c_float, ctypes.c_float, c_int, c_void_p]),
+    "pq_mlp_forward": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    "pq_mlp_backward": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                c_int, c_void_p]),
+    "pq_mlp_adam_multi": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float,
+                                  ctypes.c_float, ctypes.c_float, ctypes.c_float, c_int, c_void_p]),
     "pq_scf_set_observer": (c_int, [SCF_OBSERVER, c_void_p, c_double, c_void_p, c_void_p]),
     "pq_eigh_refine_work": (ctypes.c_longlong, [c_int]),
     "pq_eigh_batched": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p]),

@@ -2478,10 +2478,50 @@ extern "C" int pq_mlp_mse(const float* Y, const float* T, const float* mask, flo
     return 0;
 }
 
+extern "C" int pq_mlp_forward(int nlayer, const int* dims, const float* X, const float* const* W,
+                              const float* const* b, float* const* A, int B, void* stream)
+{
+    if (nlayer <= 0 || nlayer > MLP_MAX_LAYERS) return fail("pq_mlp_forward: 1 to 8 layers");
+    if (!dims || !X || !W || !b || !A || !A[nlayer - 1]) return fail("pq_mlp_forward: null argument");
+    for (int l = 0; l < nlayer; ++l)
+        if (!W[l] || !b[l]) return fail("pq_mlp_forward: null argument");
+    const int rc = mlp_forward(nlayer, dims, X, W, b, A, B, (hipStream_t)stream);
+    if (rc == -2) return fail("pq_mlp_forward: layers wider than 448 need every output buffer");
+    if (rc) return fail("pq_mlp_forward: launch failed");
+    return 0;
+}
+
+extern "C" int pq_mlp_backward(int nlayer, const int* dims, const float* X, const float* const* A,
+                               const float* const* W, const float* dY, float* const* dZ, float* const* dW,
+                               float* const* db, int B, void* stream)
+{
+    if (nlayer <= 0 || nlayer > MLP_MAX_LAYERS) return fail("pq_mlp_backward: 1 to 8 layers");
+    if (!dims || !X || !A || !W || !dY || !dZ || !dW || !db) return fail("pq_mlp_backward: null argument");
+    for (int l = 0; l < nlayer; ++l)
+        if (!W[l] || !dW[l] || !db[l] || (l + 1 < nlayer && (!A[l] || !dZ[l])))
+            return fail("pq_mlp_backward: null argument");
+    if (mlp_backward(nlayer, dims, X, A, W, dY, dZ, dW, db, B, (hipStream_t)stream))
+        return fail("pq_mlp_backward: launch failed");
+    return 0;
+}
+
 extern "C" int pq_mlp_adam(float* p, const float* g, float* m, float* v, long long n, float lr, float b1, float b2,
                            float eps, int step, void* stream)
 {
     if (!p || !g || !m || !v) return fail("pq_mlp_adam: null argument");
-    if (mlp_adam(p, g, m, v, n, lr, b1, b2, eps, step, (hipStream_t)stream)) return fail("pq_mlp_adam: launch failed");
+    if (mlp_adam(1, &p, &g, &m, &v, &n, lr, b1, b2, eps, step, (hipStream_t)stream))
+        return fail("pq_mlp_adam: launch failed");
+    return 0;
+}
+
+extern "C" int pq_mlp_adam_multi(int nt, float* const* p, const float* const* g, float* const* m, float* const* v,
+                                 const long long* n, float lr, float b1, float b2, float eps, int step, void* stream)
+{
+    if (nt <= 0 || nt > MLP_MAX_TENSORS) return fail("pq_mlp_adam_multi: 1 to 16 tensors");
+    if (!p || !g || !m || !v || !n) return fail("pq_mlp_adam_multi: null argument");
+    for (int t = 0; t < nt; ++t)
+        if (!p[t] || !g[t] || !m[t] || !v[t]) return fail("pq_mlp_adam_multi: null argument");
+    if (mlp_adam(nt, p, g, m, v, n, lr, b1, b2, eps, step, (hipStream_t)stream))
+        return fail("pq_mlp_adam_multi: launch failed");
     return 0;
 }

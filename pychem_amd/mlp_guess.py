@@ -3,8 +3,8 @@ atom pair to that pair's block of the alpha density matrix.
 
 No reference counterpart: the reference starts from the core Hamiltonian
 (Methods/hartree_fock.py:55-57).  The network is trained and evaluated with
-the library's own FP32 kernels (pq_mlp_linear_fwd / _bwd, pq_mlp_mse,
-pq_mlp_adam); torch only provides device buffers.
+the library's own FP32 kernels (pq_mlp_forward / _backward, pq_mlp_mse,
+pq_mlp_adam_multi); torch only provides device buffers.
 
 Density blocks are not rotation invariant, so each block is learned in a
 local frame of its atom pair and rotated back:
@@ -325,6 +325,19 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+# widest layer of the one-launch network kernels (pq_mlp_forward)
+FUSED_WIDTH = 448
+
+
+def _ptrs(tensors):
+    """Host array of device pointers (None: NULL)."""
+    return (ctypes.c_void_p * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
+
+
+def _dims(dims):
+    return (ctypes.c_int * len(dims))(*dims)
+
+
 class MLP:
     """Input -> 3 x (128, tanh) -> linear output, FP32 on the GPU."""
 
@@ -346,35 +359,23 @@ class MLP:
         return self.W + self.b
 
     def forward(self, X, keep=False):
-        L = _lib.lib()
-        acts = [X]
-        zs = []
-        for i in range(4):
-            B, I, O = X.shape[0], self.dims[i], self.dims[i + 1]
-            Z = torch.empty((B, O), dtype=torch.float32, device=X.device)
-            A = torch.empty_like(Z)
-            act = 1 if i < 3 else 0
-            check(L.pq_mlp_linear_fwd(_ptr(acts[-1]), _ptr(self.W[i]), _ptr(self.b[i]), _ptr(Z), _ptr(A),
-                                      B, I, O, act, _stream()), "pq_mlp_linear_fwd")
-            zs.append(Z)
-            acts.append(A)
-        return (acts[-1], acts) if keep else acts[-1]
+        B, last = X.shape[0], len(self.W) - 1
+        wide = max(self.dims) > FUSED_WIDTH      # such layers go one launch each, through buffers of their own
+        outs = [torch.empty((B, self.dims[i + 1]), dtype=torch.float32, device=X.device)
+                if keep or wide or i == last else None for i in range(last + 1)]
+        check(_lib.lib().pq_mlp_forward(last + 1, _dims(self.dims), _ptr(X), _ptrs(self.W), _ptrs(self.b), _ptrs(outs),
+                                        B, _stream()), "pq_mlp_forward")
+        return (outs[-1], [X] + outs) if keep else outs[-1]
 
     def backward(self, acts, dY):
         """Gradients of the parameters given dLoss/dY; returns (gW, gb)."""
-        L = _lib.lib()
+        n = len(self.W)
+        B = acts[0].shape[0]
         gW = [torch.empty_like(w) for w in self.W]
         gb = [torch.empty_like(b) for b in self.b]
-        dA = dY
-        for i in reversed(range(4)):
-            B, I, O = acts[i].shape[0], self.dims[i], self.dims[i + 1]
-            dZ = torch.empty((B, O), dtype=torch.float32, device=dY.device)
-            dX = torch.empty((B, I), dtype=torch.float32, device=dY.device) if i > 0 else None
-            act = 1 if i < 3 else 0
-            check(L.pq_mlp_linear_bwd(_ptr(acts[i]), _ptr(self.W[i]), _ptr(acts[i + 1]), _ptr(dA), _ptr(dZ),
-                                      _ptr(dX) if dX is not None else None, _ptr(gW[i]), _ptr(gb[i]),
-                                      B, I, O, act, _stream()), "pq_mlp_linear_bwd")
-            dA = dX
+        dZ = [torch.empty((B, self.dims[i + 1]), dtype=torch.float32, device=dY.device) for i in range(n - 1)]
+        check(_lib.lib().pq_mlp_backward(n, _dims(self.dims), _ptr(acts[0]), _ptrs(acts[1:]), _ptrs(self.W), _ptr(dY),
+                                         _ptrs(dZ + [None]), _ptrs(gW), _ptrs(gb), B, _stream()), "pq_mlp_backward")
         return gW, gb
 
     def loss_grad(self, Y, T):
@@ -388,9 +389,10 @@ class MLP:
     def adam(self, gW, gb, lr=1e-3):
         L = _lib.lib()
         self.step += 1
-        for p, g, m, v in zip(self.params(), gW + gb, self.m, self.v):
-            check(L.pq_mlp_adam(_ptr(p), _ptr(g), _ptr(m), _ptr(v), p.numel(), lr, 0.9, 0.999, 1e-8, self.step,
-                                _stream()), "pq_mlp_adam")
+        ps = self.params()
+        sizes = (ctypes.c_longlong * len(ps))(*[p.numel() for p in ps])
+        check(L.pq_mlp_adam_multi(len(ps), _ptrs(ps), _ptrs(gW + gb), _ptrs(self.m), _ptrs(self.v), sizes, lr, 0.9,
+                                  0.999, 1e-8, self.step, _stream()), "pq_mlp_adam_multi")
 
     def state(self):
         d = {"W%d" % i: w.cpu().numpy() for i, w in enumerate(self.W)}
