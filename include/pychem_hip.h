@@ -202,8 +202,7 @@ int pq_gemm_f64(int ta, int tb, int M, int N, int K, double alpha, const double*
                 long long sA, const double* B, long long ldb, long long sB, double beta, double* C,
                 long long ldc, long long sC, int batch, void* stream);
 /* pq_gemm_f64's product with split-BF16 matrix-core products: every FP64
- * operand element is rounded to FP32 and split into hi = bf16(x) and
- * lo = bf16(x - hi); a*b = hi*hi + hi*lo + lo*hi, accumulated in FP32,
+ * operand element x is split into hi = bf16(x) and lo = bf16(fp32(x) - hi); a*b = hi*hi + hi*lo + lo*hi, accumulated in FP32,
  * written as FP64 (relative error ~1e-5 per product).  No reference
  * counterpart: the reference's MP2 transform is FP64 numpy. */
 int pq_gemm_bf16x3(int ta, int tb, int M, int N, int K, double alpha, const double* A, long long lda,
@@ -211,10 +210,10 @@ int pq_gemm_bf16x3(int ta, int tb, int M, int N, int K, double alpha, const doub
                    long long ldc, long long sC, int batch, void* stream);
 
 /* AO->MO transform (ia|jb) = sum C1_mi C1v_na C2_lj C2v_sb (mn|ls) from the
- * stored ERIs, by quarter transforms over slabs of lam (at most
- * max_slab_bytes of dense AO integrals at a time; <= 0: slabs sized to half
- * of the free device memory, so that the stored quartets are read as few
- * times as possible).
+ * stored ERIs, by quarter transforms over the packed function pairs (lam sig),
+ * lam >= sig, in slabs (at most max_slab_bytes of AO integrals at a time, one
+ * pair at least; <= 0: slabs sized to half of the free device memory, so that
+ * the stored quartets are read as few times as possible).
  * C matrices are row-major over Cartesian AOs: Co1[ncart][o1] etc.
  * ovov_dev is [o1][v1][o2][v2].  precision 0: FP64 matrix-core products;
  * 1: the pq_gemm_bf16x3 products (FP32 accumulation).  Replaces the O(N^6)

@@ -114,6 +114,24 @@ struct ScatterArgs {
     int nq, n, l0, lc;
 };
 
+template <typename real>
+struct PairScatterArgs {
+    const int2* quartets;
+    const PairHdr* pairs;
+    const int* pair_base;    // first packed index of each shell pair
+    const real* vals;
+    double* out;             // out[P - p0][Q], P in [p0, p0 + rows), Q in [0, np)
+    long long p0, rows, np;
+    int nq;
+};
+
+// index of functions (i, j) of a shell pair within its packed block: all
+// N1 x N2 of two shells, i >= j of one shell with itself
+__host__ __device__ __forceinline__ int pair_component(bool same, int n2, int i, int j)
+{
+    return same ? i * (i + 1) / 2 + j : i * n2 + j;
+}
+
 // --------------------------------------------------------------------------
 // Boys function F_m(T), m = 0..L
 //   T < 36: 9-term Taylor expansion of F_L about the nearest grid point

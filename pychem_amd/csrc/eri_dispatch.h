@@ -6,10 +6,12 @@ void eri_run_0000_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_0000_d();
 void jk_run_0000_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_0000_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_0000_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_0000_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_0000_f();
 void jk_run_0000_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_0000_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_0000_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_0000_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_0000_mix();
 void eri_run_0000_s(const EriArgs<double>&, hipStream_t);
@@ -18,10 +20,12 @@ void eri_run_1000_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_1000_d();
 void jk_run_1000_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_1000_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_1000_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_1000_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1000_f();
 void jk_run_1000_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_1000_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_1000_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_1000_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1000_mix();
 void eri_run_1000_s(const EriArgs<double>&, hipStream_t);
@@ -30,10 +34,12 @@ void eri_run_1010_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_1010_d();
 void jk_run_1010_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_1010_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_1010_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_1010_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1010_f();
 void jk_run_1010_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_1010_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_1010_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_1010_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1010_mix();
 void eri_run_1010_s(const EriArgs<double>&, hipStream_t);
@@ -42,10 +48,12 @@ void eri_run_1100_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_1100_d();
 void jk_run_1100_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_1100_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_1100_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_1100_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1100_f();
 void jk_run_1100_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_1100_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_1100_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_1100_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1100_mix();
 void eri_run_1100_s(const EriArgs<double>&, hipStream_t);
@@ -54,10 +62,12 @@ void eri_run_1110_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_1110_d();
 void jk_run_1110_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_1110_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_1110_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_1110_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1110_f();
 void jk_run_1110_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_1110_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_1110_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_1110_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1110_mix();
 void eri_run_1110_s(const EriArgs<double>&, hipStream_t);
@@ -66,10 +76,12 @@ void eri_run_1111_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_1111_d();
 void jk_run_1111_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_1111_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_1111_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_1111_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1111_f();
 void jk_run_1111_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_1111_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_1111_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_1111_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_1111_mix();
 void eri_run_1111_s(const EriArgs<double>&, hipStream_t);
@@ -78,10 +90,12 @@ void eri_run_2000_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2000_d();
 void jk_run_2000_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2000_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2000_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2000_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2000_f();
 void jk_run_2000_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2000_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2000_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2000_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2000_mix();
 void eri_run_2000_s(const EriArgs<double>&, hipStream_t);
@@ -90,10 +104,12 @@ void eri_run_2010_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2010_d();
 void jk_run_2010_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2010_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2010_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2010_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2010_f();
 void jk_run_2010_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2010_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2010_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2010_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2010_mix();
 void eri_run_2010_s(const EriArgs<double>&, hipStream_t);
@@ -102,10 +118,12 @@ void eri_run_2011_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2011_d();
 void jk_run_2011_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2011_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2011_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2011_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2011_f();
 void jk_run_2011_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2011_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2011_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2011_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2011_mix();
 void eri_run_2011_s(const EriArgs<double>&, hipStream_t);
@@ -114,10 +132,12 @@ void eri_run_2020_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2020_d();
 void jk_run_2020_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2020_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2020_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2020_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2020_f();
 void jk_run_2020_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2020_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2020_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2020_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2020_mix();
 void eri_run_2020_s(const EriArgs<double>&, hipStream_t);
@@ -126,10 +146,12 @@ void eri_run_2100_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2100_d();
 void jk_run_2100_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2100_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2100_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2100_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2100_f();
 void jk_run_2100_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2100_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2100_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2100_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2100_mix();
 void eri_run_2100_s(const EriArgs<double>&, hipStream_t);
@@ -138,10 +160,12 @@ void eri_run_2110_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2110_d();
 void jk_run_2110_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2110_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2110_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2110_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2110_f();
 void jk_run_2110_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2110_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2110_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2110_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2110_mix();
 void eri_run_2110_s(const EriArgs<double>&, hipStream_t);
@@ -150,10 +174,12 @@ void eri_run_2111_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2111_d();
 void jk_run_2111_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2111_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2111_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2111_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2111_f();
 void jk_run_2111_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2111_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2111_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2111_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2111_mix();
 void eri_run_2111_s(const EriArgs<double>&, hipStream_t);
@@ -162,10 +188,12 @@ void eri_run_2120_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2120_d();
 void jk_run_2120_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2120_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2120_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2120_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2120_f();
 void jk_run_2120_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2120_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2120_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2120_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2120_mix();
 void eri_run_2120_s(const EriArgs<double>&, hipStream_t);
@@ -174,10 +202,12 @@ void eri_run_2121_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2121_d();
 void jk_run_2121_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2121_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2121_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2121_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2121_f();
 void jk_run_2121_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2121_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2121_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2121_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2121_mix();
 void eri_run_2121_s(const EriArgs<double>&, hipStream_t);
@@ -186,10 +216,12 @@ void eri_run_2200_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2200_d();
 void jk_run_2200_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2200_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2200_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2200_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2200_f();
 void jk_run_2200_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2200_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2200_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2200_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2200_mix();
 void eri_run_2200_s(const EriArgs<double>&, hipStream_t);
@@ -198,10 +230,12 @@ void eri_run_2210_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2210_d();
 void jk_run_2210_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2210_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2210_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2210_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2210_f();
 void jk_run_2210_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2210_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2210_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2210_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2210_mix();
 void eri_run_2210_s(const EriArgs<double>&, hipStream_t);
@@ -210,10 +244,12 @@ void eri_run_2211_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2211_d();
 void jk_run_2211_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2211_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2211_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2211_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2211_f();
 void jk_run_2211_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2211_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2211_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2211_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2211_mix();
 void eri_run_2211_s(const EriArgs<double>&, hipStream_t);
@@ -222,10 +258,12 @@ void eri_run_2220_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2220_d();
 void jk_run_2220_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2220_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2220_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2220_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2220_f();
 void jk_run_2220_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2220_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2220_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2220_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2220_mix();
 void eri_run_2220_s(const EriArgs<double>&, hipStream_t);
@@ -234,10 +272,12 @@ void eri_run_2221_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2221_d();
 void jk_run_2221_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2221_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2221_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2221_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2221_f();
 void jk_run_2221_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2221_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2221_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2221_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2221_mix();
 void eri_run_2221_s(const EriArgs<double>&, hipStream_t);
@@ -246,10 +286,12 @@ void eri_run_2222_d(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2222_d();
 void jk_run_2222_d(const JkArgs<double>&, hipStream_t);
 void scatter_run_2222_d(const ScatterArgs<double>&, hipStream_t);
+void pairscatter_run_2222_d(const PairScatterArgs<double>&, hipStream_t);
 void eri_run_2222_f(const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2222_f();
 void jk_run_2222_f(const JkArgs<float>&, hipStream_t);
 void scatter_run_2222_f(const ScatterArgs<float>&, hipStream_t);
+void pairscatter_run_2222_f(const PairScatterArgs<float>&, hipStream_t);
 void eri_run_2222_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);
 size_t eri_scratch_2222_mix();
 void eri_run_2222_s(const EriArgs<double>&, hipStream_t);
@@ -383,3 +425,11 @@ static void (*const scatter_table_f[ERI_NCLASS])(const ScatterArgs<float>&, hipS
 };
 template <typename real> static inline void scatter_launch(int cls, const ScatterArgs<real>& a, hipStream_t st)
 { if (sizeof(real) == 8) scatter_table_d[cls]((const ScatterArgs<double>&)a, st); else scatter_table_f[cls]((const ScatterArgs<float>&)a, st); }
+static void (*const pairscatter_table_d[ERI_NCLASS])(const PairScatterArgs<double>&, hipStream_t) = {
+  pairscatter_run_0000_d, pairscatter_run_1000_d, pairscatter_run_1010_d, pairscatter_run_1100_d, pairscatter_run_1110_d, pairscatter_run_1111_d, pairscatter_run_2000_d, pairscatter_run_2010_d, pairscatter_run_2011_d, pairscatter_run_2020_d, pairscatter_run_2100_d, pairscatter_run_2110_d, pairscatter_run_2111_d, pairscatter_run_2120_d, pairscatter_run_2121_d, pairscatter_run_2200_d, pairscatter_run_2210_d, pairscatter_run_2211_d, pairscatter_run_2220_d, pairscatter_run_2221_d, pairscatter_run_2222_d
+};
+static void (*const pairscatter_table_f[ERI_NCLASS])(const PairScatterArgs<float>&, hipStream_t) = {
+  pairscatter_run_0000_f, pairscatter_run_1000_f, pairscatter_run_1010_f, pairscatter_run_1100_f, pairscatter_run_1110_f, pairscatter_run_1111_f, pairscatter_run_2000_f, pairscatter_run_2010_f, pairscatter_run_2011_f, pairscatter_run_2020_f, pairscatter_run_2100_f, pairscatter_run_2110_f, pairscatter_run_2111_f, pairscatter_run_2120_f, pairscatter_run_2121_f, pairscatter_run_2200_f, pairscatter_run_2210_f, pairscatter_run_2211_f, pairscatter_run_2220_f, pairscatter_run_2221_f, pairscatter_run_2222_f
+};
+template <typename real> static inline void pairscatter_launch(int cls, const PairScatterArgs<real>& a, hipStream_t st)
+{ if (sizeof(real) == 8) pairscatter_table_d[cls]((const PairScatterArgs<double>&)a, st); else pairscatter_table_f[cls]((const PairScatterArgs<float>&)a, st); }

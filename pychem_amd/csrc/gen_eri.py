@@ -571,6 +571,11 @@ def main():
             jsrc.append("void scatter_run_%s_%s(const ScatterArgs<%s>& a, hipStream_t st)" % (tag, rn, rt))
             jsrc.append("{ hipLaunchKernelGGL((scatter_kernel<%d, %d, %d, %d, %s>), dim3((unsigned)((a.nq * %dLL + 255) / 256)), "
                         "dim3(256), 0, st, a); }" % (la, lb, lc, ld, rt, ncomp))
+            jsrc.append("void pairscatter_run_%s_%s(const PairScatterArgs<%s>& a, hipStream_t st)" % (tag, rn, rt))
+            n12 = (la + 1) * (la + 2) // 2 * ((lb + 1) * (lb + 2) // 2)
+            jsrc.append("{ hipLaunchKernelGGL((pair_scatter_kernel<%d, %d, %d, %d, %s>), dim3((a.nq + 255) / 256, "
+                        "%d / PairScatterSplit<%d, %d>::AB), dim3(256), 0, st, a); }"
+                        % (la, lb, lc, ld, rt, n12, n12, ncomp // n12))
         _write_if_changed(os.path.join(gdir, "cls_%s.hip" % tag), "\n".join(src) + "\n")
         ta, tb, nt = jk_tile(la, lb, lc, ld)
         jsrc.append("void jktile_run_%s(const JkTileArgs& a, int block, hipStream_t st)" % tag)
@@ -649,6 +654,7 @@ def main():
             d.append("size_t eri_scratch_%s_%s();" % (tag, rn))
             d.append("void jk_run_%s_%s(const JkArgs<%s>&, hipStream_t);" % (tag, rn, rt))
             d.append("void scatter_run_%s_%s(const ScatterArgs<%s>&, hipStream_t);" % (tag, rn, rt))
+            d.append("void pairscatter_run_%s_%s(const PairScatterArgs<%s>&, hipStream_t);" % (tag, rn, rt))
         d.append("void eri_run_%s_mix(const EriArgs<double>&, const EriArgs<float>&, hipStream_t);" % tag)
         d.append("size_t eri_scratch_%s_mix();" % tag)
         d.append("void eri_run_%s_s(const EriArgs<double>&, hipStream_t);" % tag)
@@ -695,7 +701,8 @@ def main():
     d.append("static void (*const eri_table_mix[ERI_NCLASS])(const EriArgs<double>&, const EriArgs<float>&, hipStream_t) = {")
     d.append("  " + ", ".join("eri_run_%d%d%d%d_mix" % (t[0], t[1], t[2], t[3]) for t in table))
     d.append("};")
-    for kname, targ in (("eri", "EriArgs"), ("jk", "JkArgs"), ("scatter", "ScatterArgs")):
+    for kname, targ in (("eri", "EriArgs"), ("jk", "JkArgs"), ("scatter", "ScatterArgs"),
+                        ("pairscatter", "PairScatterArgs")):
         for rn, rt in (("d", "double"), ("f", "float")):
             d.append("static void (*const %s_table_%s[ERI_NCLASS])(const %s<%s>&, hipStream_t) = {" % (kname, rn, targ, rt))
             d.append("  " + ", ".join("%s_run_%d%d%d%d_%s" % (kname, t[0], t[1], t[2], t[3], rn) for t in table))
