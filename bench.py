@@ -16,10 +16,9 @@ second of whole-solve wall time.  Beside it:
 * ``mixed_learned``: the same molecule with FP32 ERIs below a Schwarz bound
   product of 1e-6 and the learned (MLP) guess: time, speed-up over plain
   FP64, |dE| against it.
-* ``roofline``: the kernel with the largest share of the solve's kernel time
-  (the J/K digestion class with the most time per solve in the rocprofv3
-  trace of this command), timed live with HIP events around every launch of
-  it in the timed solves (on the stream it runs on), against 8 TB/s;
+* ``roofline``: the J/K digestion class with the most time per solve, timed
+  live in every Fock build of the timed solves (from its first block's start
+  to its last block's end, by the GPU's realtime clock), against 8 TB/s;
   ``traffic`` from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs summarised in
   profiles/pmc_traffic.json when they were taken for that kernel and
   workload; ``roofline.jk_build``: every class's digestion bytes over the
@@ -108,9 +107,10 @@ def jk_class_bytes(s, nitems, fm):
 
 
 def jk_kernel_name(cls, fm):
+    """The class's part of its group's launch (jk_group_kernel_*)."""
     la, lb, lc, ld = (int(x) for x in cls)
     ta, tb, _ = fm[cls]["jk_tile"]
-    return "jk_tile_kernel<%d, %d, %d, %d, %d, %d>" % (la, lb, lc, ld, ta, tb)
+    return "jk_tile_class<%d, %d, %d, %d, %d, %d>" % (la, lb, lc, ld, ta, tb)
 
 
 def pmc_traffic(kernel, workload_name):
@@ -496,8 +496,8 @@ def main():
     nprim = sum(s["nprim64"] + s["nprim32"] for s in stats)
     value = nq * args.steps / wall
 
-    # the dominant kernel: the J/K digestion class with the most time per
-    # solve, every launch of it in the timed solves timed on its own stream
+    # the dominant J/K digestion class: the most time per solve, every Fock
+    # build of the timed solves timed
     sums = sum(x[2][0] for x in results)
     launches = sum(x[2][1] for x in results)
     nitems = results[-1][2][2]

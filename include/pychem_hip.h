@@ -114,11 +114,12 @@ int pq_set_timing(pq_basis* b, int on);
  * side streams), of the whole pass (eri_pass_ms, on the caller's stream) and
  * of the last pq_jk call.  Outputs may be NULL. */
 int pq_get_timings(pq_basis* b, double* eri_ms, double* jk_ms, double* eri_pass_ms);
-/* Per-class J/K digestion kernel times summed over the J/K calls made with
- * timing on (pq_jk, pq_jk_general and the J/K of pq_scf_run; HIP events on
- * the stream each class ran on), the number of timed launches and each
- * class's J/K work items, ERI_NCLASS entries each (any may be NULL); reset
- * != 0 clears the sums.  No reference counterpart (measurement). */
+/* Per-class J/K digestion times summed over the J/K calls made with timing
+ * on (pq_jk, pq_jk_general and the J/K of pq_scf_run): from the start of the
+ * class's first block to the end of its last, by the GPU's realtime clock (the
+ * classes share launches); the number of calls and each class's J/K work
+ * items, ERI_NCLASS entries each (any may be NULL); reset != 0 clears the
+ * sums.  Waits for the device.  No reference counterpart (measurement). */
 int pq_jk_class_times(pq_basis* b, double* sum_ms, long long* launches, long long* nitems, int reset);
 /* Recompute one class of the stored ERIs: cls in [0, pq_eri_nclass()),
  * w = 0 for the FP64 list, 1 for the FP32 list. */
@@ -167,8 +168,8 @@ int pq_jk_general_noalloc(pq_basis* b, const double* Dj_dev, const double* Dk_de
 int pq_jk_set_params(pq_basis* b, int cls, int run_len, int grid, void* stream);
 int pq_jk_class(pq_basis* b, int cls, int part, const double* Dj_dev, const double* Dk_dev, double* J_dev,
                 double* K_dev, int* nitems, void* stream);
-/* Number of streams (1..4, default 4) that pq_jk spreads its class launches
- * over: the caller's stream and up to three side streams forked from it and
+/* Number of streams (1..4, default 4) that pq_jk spreads its launches over when
+ * the stored integrals exceed 400 MB (one below): the caller's stream and up to three side streams forked from it and
  * joined back to it (no reference counterpart: the reference digests one
  * quartet at a time on the host). */
 int pq_jk_set_streams(pq_basis* b, int nstreams);

@@ -347,56 +347,42 @@ static size_t (*const eri_scratch_table_mix[ERI_NCLASS])() = {
 static size_t (*const eri_scratch_table_s[ERI_NCLASS])() = {
   eri_scratch_0000_s, eri_scratch_1000_s, eri_scratch_1010_s, eri_scratch_1100_s, eri_scratch_1110_s, eri_scratch_1111_s, eri_scratch_2000_s, eri_scratch_2010_s, eri_scratch_2011_s, eri_scratch_2020_s, eri_scratch_2100_s, eri_scratch_2110_s, eri_scratch_2111_s, eri_scratch_2120_s, eri_scratch_2121_s, eri_scratch_2200_s, eri_scratch_2210_s, eri_scratch_2211_s, eri_scratch_2220_s, eri_scratch_2221_s, eri_scratch_2222_s
 };
-// tiled J/K: bra tile TA x TB, tiles per quartet, LDS doubles per basis function (2 (TA + TB))
+// tiled J/K: bra tile TA x TB, tiles per quartet, LDS doubles per basis function
 static const int jk_tile_table[ERI_NCLASS][4] = {
-  {1, 1, 1, 4},
-  {3, 1, 1, 8},
-  {3, 1, 1, 8},
-  {3, 3, 1, 12},
-  {3, 3, 1, 12},
-  {3, 3, 1, 12},
+  {1, 1, 1, 6},
+  {3, 1, 1, 10},
+  {3, 1, 1, 10},
+  {3, 3, 1, 14},
+  {3, 3, 1, 14},
+  {3, 3, 1, 14},
   {6, 1, 1, 14},
   {6, 1, 1, 14},
   {6, 1, 1, 14},
   {6, 1, 1, 14},
   {6, 3, 1, 18},
   {6, 3, 1, 18},
-  {3, 3, 2, 12},
+  {3, 3, 2, 14},
   {6, 3, 1, 18},
-  {3, 3, 2, 12},
+  {3, 3, 2, 14},
   {3, 6, 2, 18},
   {3, 6, 2, 18},
-  {3, 3, 4, 12},
+  {3, 3, 4, 14},
   {3, 6, 2, 18},
-  {3, 3, 4, 12},
-  {2, 2, 9, 8},
+  {3, 3, 4, 14},
+  {2, 2, 9, 10},
 };
-void jktile_run_0000(const JkTileArgs&, int, hipStream_t);
-void jktile_run_1000(const JkTileArgs&, int, hipStream_t);
-void jktile_run_1010(const JkTileArgs&, int, hipStream_t);
-void jktile_run_1100(const JkTileArgs&, int, hipStream_t);
-void jktile_run_1110(const JkTileArgs&, int, hipStream_t);
-void jktile_run_1111(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2000(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2010(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2011(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2020(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2100(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2110(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2111(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2120(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2121(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2200(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2210(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2211(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2220(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2221(const JkTileArgs&, int, hipStream_t);
-void jktile_run_2222(const JkTileArgs&, int, hipStream_t);
-static void (*const jktile_table[ERI_NCLASS])(const JkTileArgs&, int, hipStream_t) = {
-  jktile_run_0000, jktile_run_1000, jktile_run_1010, jktile_run_1100, jktile_run_1110, jktile_run_1111, jktile_run_2000, jktile_run_2010, jktile_run_2011, jktile_run_2020, jktile_run_2100, jktile_run_2110, jktile_run_2111, jktile_run_2120, jktile_run_2121, jktile_run_2200, jktile_run_2210, jktile_run_2211, jktile_run_2220, jktile_run_2221, jktile_run_2222
+// J/K launch groups
+#define JK_NGROUP 4
+static const int jk_group_table[ERI_NCLASS] = {
+  0, 0, 0, 2, 2, 2, 1, 1, 2, 1, 3, 3, 2, 3, 2, 3, 3, 2, 3, 2, 2
 };
-static inline void jktile_launch(int cls, const JkTileArgs& a, int block, hipStream_t st)
-{ jktile_table[cls](a, block, st); }
+void jk_group_run_0(const JkGroupArgs&, int, int, size_t, hipStream_t);
+void jk_group_run_1(const JkGroupArgs&, int, int, size_t, hipStream_t);
+void jk_group_run_2(const JkGroupArgs&, int, int, size_t, hipStream_t);
+void jk_group_run_3(const JkGroupArgs&, int, int, size_t, hipStream_t);
+static void (*const jk_group_run[JK_NGROUP])(const JkGroupArgs&, int, int, size_t, hipStream_t) = {
+  jk_group_run_0, jk_group_run_1, jk_group_run_2, jk_group_run_3
+};
 // both lists of a class in one launch
 static void (*const eri_table_mix[ERI_NCLASS])(const EriArgs<double>&, const EriArgs<float>&, hipStream_t) = {
   eri_run_0000_mix, eri_run_1000_mix, eri_run_1010_mix, eri_run_1100_mix, eri_run_1110_mix, eri_run_1111_mix, eri_run_2000_mix, eri_run_2010_mix, eri_run_2011_mix, eri_run_2020_mix, eri_run_2100_mix, eri_run_2110_mix, eri_run_2111_mix, eri_run_2120_mix, eri_run_2121_mix, eri_run_2200_mix, eri_run_2210_mix, eri_run_2211_mix, eri_run_2220_mix, eri_run_2221_mix, eri_run_2222_mix

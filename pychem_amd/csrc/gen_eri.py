@@ -467,6 +467,18 @@ def jk_tile(la, lb, lc, ld, budget=72):
     return ta, tb, (n1 // ta) * (n2 // tb)
 
 
+# J/K launch groups by rows staged (TA + TB), which also orders the classes by
+# the registers their digestion takes (86, 128, 207 and 230 at most)
+JK_GROUPS = [(0, 4), (7, 7), (5, 6), (8, 99)]
+
+
+def jk_group(la, lb, lc, ld):
+    ta, tb, _ = jk_tile(la, lb, lc, ld)
+    if (la, lb, lc, ld) in ((2, 2, 2, 2), (2, 0, 1, 1)):
+        return 2          # few rows, but the registers of the 3 x 3 tiles
+    return next(g for g, (lo, hi) in enumerate(JK_GROUPS) if lo <= ta + tb <= hi)
+
+
 # classes whose kernels spill (scratch) with this generator's code would
 # share one fused launch on the caller's stream (scratch is sized per hardware
 # queue); with the output split above none does
@@ -577,11 +589,26 @@ def main():
                         "%d / PairScatterSplit<%d, %d>::AB), dim3(256), 0, st, a); }"
                         % (la, lb, lc, ld, rt, n12, n12, ncomp // n12))
         _write_if_changed(os.path.join(gdir, "cls_%s.hip" % tag), "\n".join(src) + "\n")
-        ta, tb, nt = jk_tile(la, lb, lc, ld)
-        jsrc.append("void jktile_run_%s(const JkTileArgs& a, int block, hipStream_t st)" % tag)
-        jsrc.append("{ hipLaunchKernelGGL((jk_tile_kernel<%d, %d, %d, %d, %d, %d>), dim3(a.grid, %d), dim3(block), "
-                    "sizeof(double) * %d * a.nmax, st, a); }" % (la, lb, lc, ld, ta, tb, nt, 2 * (ta + tb)))
         _write_if_changed(os.path.join(gdir, "jk_%s.hip" % tag), "\n".join(jsrc) + "\n")
+    # J/K launch groups: classes whose kernels need about the same registers
+    # and LDS rows in one kernel
+    for g in range(len(JK_GROUPS)):
+        js = ["// generated by gen_eri.py -- do not edit", '#include "../jk_common.h"',
+              "__global__ void __launch_bounds__(256, 2) jk_group_kernel_%d(const JkGroupArgs g)" % g, "{",
+              "  extern __shared__ double lds[];", "  const int s = jk_group_slot(g);",
+              "  const JkClassArgs& a = g.c[s];", "  const int local = blockIdx.x - a.block0;",
+              "  jk_clock(g, a.cls, 0);", "  switch (a.cls) {"]
+        for k, t in enumerate(table):
+            la, lb, lc, ld = t[:4]
+            if jk_group(la, lb, lc, ld) != g:
+                continue
+            ta, tb, nt = jk_tile(la, lb, lc, ld)
+            js.append("  case %d: jk_tile_class<%d, %d, %d, %d, %d, %d>(g, a, local, lds); break;"
+                      % (k, la, lb, lc, ld, ta, tb))
+        js += ["  default: break;", "  }", "  jk_clock(g, a.cls, 1);", "}",
+               "void jk_group_run_%d(const JkGroupArgs& g, int blocks, int block, size_t lds, hipStream_t st)" % g,
+               "{ hipLaunchKernelGGL(jk_group_kernel_%d, dim3(blocks), dim3(block), lds, st, g); }" % g]
+        _write_if_changed(os.path.join(gdir, "jk_group_%d.hip" % g), "\n".join(js) + "\n")
     # the heavy classes (their one-thread-per-quartet kernels use scratch)
     # in one launch: the block index selects the class, so they run side by
     # side on one queue instead of one after another
@@ -684,19 +711,23 @@ def main():
         d.append("static size_t (*const eri_scratch_table_%s[ERI_NCLASS])() = {" % rn)
         d.append("  " + ", ".join("eri_scratch_%d%d%d%d_%s" % (t[0], t[1], t[2], t[3], rn) for t in table))
         d.append("};")
-    d.append("// tiled J/K: bra tile TA x TB, tiles per quartet, LDS doubles per basis function (2 (TA + TB))")
+    d.append("// tiled J/K: bra tile TA x TB, tiles per quartet, LDS doubles per basis function")
     d.append("static const int jk_tile_table[ERI_NCLASS][4] = {")
     for la, lb, lc, ld, ncomp, X, Y, nbody in table:
         ta, tb, nt = jk_tile(la, lb, lc, ld)
-        d.append("  {%d, %d, %d, %d}," % (ta, tb, nt, 2 * (ta + tb)))
+        d.append("  {%d, %d, %d, %d}," % (ta, tb, nt, 2 * ((ta + tb) | 1)))
     d.append("};")
-    for la, lb, lc, ld, ncomp, X, Y, nbody in table:
-        d.append("void jktile_run_%d%d%d%d(const JkTileArgs&, int, hipStream_t);" % (la, lb, lc, ld))
-    d.append("static void (*const jktile_table[ERI_NCLASS])(const JkTileArgs&, int, hipStream_t) = {")
-    d.append("  " + ", ".join("jktile_run_%d%d%d%d" % (t[0], t[1], t[2], t[3]) for t in table))
+    ng = len(JK_GROUPS)
+    d.append("// J/K launch groups")
+    d.append("#define JK_NGROUP %d" % ng)
+    d.append("static const int jk_group_table[ERI_NCLASS] = {")
+    d.append("  " + ", ".join(str(jk_group(*t[:4])) for t in table))
     d.append("};")
-    d.append("static inline void jktile_launch(int cls, const JkTileArgs& a, int block, hipStream_t st)")
-    d.append("{ jktile_table[cls](a, block, st); }")
+    for g in range(ng):
+        d.append("void jk_group_run_%d(const JkGroupArgs&, int, int, size_t, hipStream_t);" % g)
+    d.append("static void (*const jk_group_run[JK_NGROUP])(const JkGroupArgs&, int, int, size_t, hipStream_t) = {")
+    d.append("  " + ", ".join("jk_group_run_%d" % g for g in range(ng)))
+    d.append("};")
     d.append("// both lists of a class in one launch")
     d.append("static void (*const eri_table_mix[ERI_NCLASS])(const EriArgs<double>&, const EriArgs<float>&, hipStream_t) = {")
     d.append("  " + ", ".join("eri_run_%d%d%d%d_mix" % (t[0], t[1], t[2], t[3]) for t in table))

@@ -147,192 +147,126 @@ struct JkTileList {
 };
 
 // Both stored lists of one class (FP64 values, and FP32 values below the
-// Schwarz split) in one launch.  A work item is a chunk of one bra pair's
-// kets: its FP64 quartets [start, end) then its FP32 quartets items32[item]
-// (the bra's FP32 kets follow its FP64 kets in bound order), digested with
-// the same staged rows.
-struct JkTileArgs {
+// Schwarz split).  A work item is a chunk of one bra pair's kets: its FP64
+// quartets [start, end) then its FP32 quartets items32[item] (the bra's FP32
+// kets follow its FP64 kets in bound order), digested with the same staged
+// rows.
+struct JkClassArgs {
     const JkItem* items;
     const int2* items32;     // FP32 quartet range per item (NULL: FP64 list only)
     JkTileList<double> l64;
     JkTileList<float> l32;
+    int nitems, grid;        // grid: blocks per bra tile (<= nitems; each strides over items when smaller)
+    int block0;              // first block of the class in its launch
+    int cls;
+};
+
+// Several classes in one launch (jk_group_kernel_*): a Fock build is a handful
+// of launches instead of one per class.  clock (NULL: off): per class the
+// earliest start and latest end of its blocks in ticks of the realtime clock.
+#define JK_MAXCLASS 21
+struct JkGroupArgs {
+    JkClassArgs c[JK_MAXCLASS];
+    int n;
     const MolInfo* mols;
     const double* Dj;
     const double* Dk;
     double* J;
     double* K;
-    int nmax, nitems, grid;  // grid: blocks in x (<= nitems; persistent when smaller)
+    unsigned long long* clock;
+};
+
+// The TA + TB rows lie in LDS column by column, element (row r, column c) at
+// c * JkRows::stride + r: what a quartet reads or adds at one column is one
+// address with constant offsets (and pairs of reads are one instruction), where
+// rows n apart cost an address each: with the division-free staging half the
+// vector instructions of a C20H42 build (2.45e8 -> 1.40e8), 86 registers
+// instead of 100 in the lightest group and 128 instead of 156 in the (ds| one.
+// The stride is odd, so that the columns that a wave's lanes hold spread over
+// all banks.
+template <int TA, int TB>
+struct JkRows {
+    static constexpr int count = TA + TB, stride = count | 1;
 };
 
 // The quartets [q0, q1) of one list for the current item and tile.  Quartet
 // q0 + i goes to thread (i + shift) mod blockDim: with shift = the number of
 // quartets of the FP64 range, the FP32 range continues where the FP64 range
 // ended, so that in a short item no thread takes a quartet of each list.
+//
+// Classes with at least three ket components (every ket but ss) digest one
+// (quartet, ket row c) unit per thread instead of a quartet: N3 times the
+// independent units of an item, and only one row's values in registers.  Unit
+// u of the range is row u / len, quartet q0 + u % len (consecutive lanes read
+// consecutive quartets of one row).  The K contributions of row c go to the
+// LDS rows at once, the ket J values to their own jkbuf slots.  A ket of two s
+// shells is one row.
 template <int LA, int LB, int LC, int LD, int TA, int TB, typename real>
-__device__ __forceinline__ void jk_tile_quartets(const JkTileList<real>& L, int q0, int q1, int shift,
-                                                 const double* drows, double* krows, int n,
-                                                 const double* __restrict__ Dj, double sbra,
-                                                 const double (&d12)[TA][TB], double (&j12)[TA][TB], int a0, int b0,
-                                                 int tile)
-{
-    constexpr int N2 = (LB + 1) * (LB + 2) / 2;
-    constexpr int N3 = (LC + 1) * (LC + 2) / 2, N4 = (LD + 1) * (LD + 2) / 2;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const size_t nq = L.nq;
-    const real* __restrict__ vals = L.vals;
-    double* __restrict__ jkbuf = L.jkbuf;
-    const int first = (tid - shift % nt + nt) % nt;
-    for (int q = q0 + first; q < q1; q += nt) {
-            const unsigned w = L.kets[q];
-            const int o3 = w & 0x7fff, o4 = (w >> 15) & 0x7fff;
-            double sc = sbra;
-            if ((w >> 30) & 1u) sc *= 0.5;
-            if (w >> 31) sc *= 0.5;
-            double d14[TA][N4], d24[TB][N4], k14[TA][N4], k24[TB][N4];
-#pragma unroll
-            for (int d = 0; d < N4; ++d) {
-#pragma unroll
-                for (int x = 0; x < TA; ++x) {
-                    d14[x][d] = drows[x * n + o4 + d];
-                    k14[x][d] = 0.0;
-                }
-#pragma unroll
-                for (int y = 0; y < TB; ++y) {
-                    d24[y][d] = drows[(TA + y) * n + o4 + d];
-                    k24[y][d] = 0.0;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < N3; ++c) {
-                // all loads of this ket row first (values and Dj elements), so
-                // that they are in flight together
-                // values kept in the list's own type until use: an FP32 row
-                // batch takes half the registers, so its loads still fit in
-                // flight together
-                real vv[N4][TA][TB];
-                double dj[N4];
-#pragma unroll
-                for (int d = 0; d < N4; ++d) {
-                    dj[d] = Dj[(size_t)(o3 + c) * n + o4 + d];
-#pragma unroll
-                    for (int x = 0; x < TA; ++x)
-#pragma unroll
-                        for (int y = 0; y < TB; ++y)
-                            vv[d][x][y] = vals[(size_t)((((a0 + x) * N2 + b0 + y) * N3 + c) * N4 + d) * nq + q];
-                }
-                double d13[TA], d23[TB], k13[TA], k23[TB];
-#pragma unroll
-                for (int x = 0; x < TA; ++x) {
-                    d13[x] = drows[x * n + o3 + c];
-                    k13[x] = 0.0;
-                }
-#pragma unroll
-                for (int y = 0; y < TB; ++y) {
-                    d23[y] = drows[(TA + y) * n + o3 + c];
-                    k23[y] = 0.0;
-                }
-#pragma unroll
-                for (int d = 0; d < N4; ++d) {
-                    double jcd = 0.0;
-#pragma unroll
-                    for (int x = 0; x < TA; ++x)
-#pragma unroll
-                        for (int y = 0; y < TB; ++y) {
-                            const double v = sc * (double)vv[d][x][y];
-                            j12[x][y] += dj[d] * v;
-                            jcd += d12[x][y] * v;
-                            k13[x] += d24[y][d] * v;
-                            k14[x][d] += d23[y] * v;
-                            k23[y] += d14[x][d] * v;
-                            k24[y][d] += d13[x] * v;
-                        }
-                    jkbuf[(size_t)(tile * N3 * N4 + c * N4 + d) * nq + q] = 4.0 * jcd;
-                }
-#pragma unroll
-                for (int x = 0; x < TA; ++x) atomicAdd(&krows[x * n + o3 + c], 2.0 * k13[x]);
-#pragma unroll
-                for (int y = 0; y < TB; ++y) atomicAdd(&krows[(TA + y) * n + o3 + c], 2.0 * k23[y]);
-            }
-#pragma unroll
-            for (int d = 0; d < N4; ++d) {
-#pragma unroll
-                for (int x = 0; x < TA; ++x) atomicAdd(&krows[x * n + o4 + d], 2.0 * k14[x][d]);
-#pragma unroll
-                for (int y = 0; y < TB; ++y) atomicAdd(&krows[(TA + y) * n + o4 + d], 2.0 * k24[y][d]);
-            }
-            }
-}
+struct JkUnit {
+    static constexpr int N2 = (LB + 1) * (LB + 2) / 2;
+    static constexpr int N3 = (LC + 1) * (LC + 2) / 2, N4 = (LD + 1) * (LD + 2) / 2;
+    static constexpr int RS = JkRows<TA, TB>::stride;
+    // what a unit reads from memory, all loads in flight together; values in
+    // the list's own type until use (an FP32 row takes half the registers)
+    unsigned w;
+    int q, c;
+    real vv[N4][TA][TB];
+    double dj[N4];
 
-// Classes with at least three ket components (every ket but ss)
-// digest one (quartet, ket row c) unit per thread instead of a quartet: N3
-// times the independent units of an item, and only one row's values in
-// registers.  Unit u of the range goes to row u / len, quartet q0 + u % len
-// (consecutive lanes read consecutive quartets of one row), and to thread
-// (u + shift) mod blockDim.  The K contributions of row c go to the LDS rows
-// at once, the ket J values to their own jkbuf slots as in the quartet loop.
-template <int LC, int LD>
-struct JkRowSplit {
-    static constexpr bool value = (LC + 1) * (LC + 2) / 2 * ((LD + 1) * (LD + 2) / 2) >= 3;
-};
-
-template <int LA, int LB, int LC, int LD, int TA, int TB, typename real>
-__device__ __forceinline__ void jk_tile_rows(const JkTileList<real>& L, int q0, int q1, int shift,
-                                             const double* drows, double* krows, int n,
-                                             const double* __restrict__ Dj, double sbra,
-                                             const double (&d12)[TA][TB], double (&j12)[TA][TB], int a0, int b0,
-                                             int tile)
-{
-    constexpr int N2 = (LB + 1) * (LB + 2) / 2;
-    constexpr int N3 = (LC + 1) * (LC + 2) / 2, N4 = (LD + 1) * (LD + 2) / 2;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int len = q1 - q0;
-    if (len <= 0) return;
-    const int total = N3 * len;
-    const size_t nq = L.nq;
-    const real* __restrict__ vals = L.vals;
-    double* __restrict__ jkbuf = L.jkbuf;
-    const int first = (tid - shift % nt + nt) % nt;
-    for (int u = first; u < total; u += nt) {
-        const int c = u / len;
-        const int q = q0 + (u - c * len);
-        const unsigned w = L.kets[q];
-        const int o3 = w & 0x7fff, o4 = (w >> 15) & 0x7fff;
-        double sc = sbra;
-        if ((w >> 30) & 1u) sc *= 0.5;
-        if (w >> 31) sc *= 0.5;
-        real vv[N4][TA][TB];
-        double dj[N4];
+    __device__ __forceinline__ void load(const JkTileList<real>& L, int u, int q0, int len, int n,
+                                         const double* __restrict__ Dj, int a0, int b0)
+    {
+        c = N3 > 1 ? u / len : 0;
+        q = q0 + (u - c * len);
+        const size_t nq = L.nq;
+        const real* __restrict__ vals = L.vals;
+        w = L.kets[q];
 #pragma unroll
-        for (int d = 0; d < N4; ++d) {
-            dj[d] = Dj[(size_t)(o3 + c) * n + o4 + d];
+        for (int d = 0; d < N4; ++d)
 #pragma unroll
             for (int x = 0; x < TA; ++x)
 #pragma unroll
                 for (int y = 0; y < TB; ++y)
                     vv[d][x][y] = vals[(size_t)((((a0 + x) * N2 + b0 + y) * N3 + c) * N4 + d) * nq + q];
-        }
+        const int o3 = w & 0x7fff, o4 = (w >> 15) & 0x7fff;
+#pragma unroll
+        for (int d = 0; d < N4; ++d) dj[d] = Dj[(size_t)(o3 + c) * n + o4 + d];
+    }
+
+    __device__ __forceinline__ void digest(const JkTileList<real>& L, const double* drows, double* krows, double sbra,
+                                           const double (&d12)[TA][TB], double (&j12)[TA][TB], int tile) const
+    {
+        const int o3 = w & 0x7fff, o4 = (w >> 15) & 0x7fff;
+        double sc = sbra;
+        if ((w >> 30) & 1u) sc *= 0.5;
+        if (w >> 31) sc *= 0.5;
+        const double* dc = drows + (o3 + c) * RS;
+        double* kc = krows + (o3 + c) * RS;
         double d13[TA], d23[TB], k13[TA], k23[TB];
 #pragma unroll
         for (int x = 0; x < TA; ++x) {
-            d13[x] = drows[x * n + o3 + c];
+            d13[x] = dc[x];
             k13[x] = 0.0;
         }
 #pragma unroll
         for (int y = 0; y < TB; ++y) {
-            d23[y] = drows[(TA + y) * n + o3 + c];
+            d23[y] = dc[TA + y];
             k23[y] = 0.0;
         }
+        double* __restrict__ jkbuf = L.jkbuf + (size_t)(tile * N3 * N4 + c * N4) * L.nq + q;
 #pragma unroll
         for (int d = 0; d < N4; ++d) {
+            const double* dd = drows + (o4 + d) * RS;
+            double* kd = krows + (o4 + d) * RS;
             double d14[TA], d24[TB], k14[TA], k24[TB];
 #pragma unroll
             for (int x = 0; x < TA; ++x) {
-                d14[x] = drows[x * n + o4 + d];
+                d14[x] = dd[x];
                 k14[x] = 0.0;
             }
 #pragma unroll
             for (int y = 0; y < TB; ++y) {
-                d24[y] = drows[(TA + y) * n + o4 + d];
+                d24[y] = dd[TA + y];
                 k24[y] = 0.0;
             }
             double jcd = 0.0;
@@ -348,61 +282,52 @@ __device__ __forceinline__ void jk_tile_rows(const JkTileList<real>& L, int q0, 
                     k23[y] += d14[x] * v;
                     k24[y] += d13[x] * v;
                 }
-            jkbuf[(size_t)(tile * N3 * N4 + c * N4 + d) * nq + q] = 4.0 * jcd;
+            jkbuf[(size_t)d * L.nq] = 4.0 * jcd;
 #pragma unroll
-            for (int x = 0; x < TA; ++x) atomicAdd(&krows[x * n + o4 + d], 2.0 * k14[x]);
+            for (int x = 0; x < TA; ++x) atomicAdd(&kd[x], 2.0 * k14[x]);
 #pragma unroll
-            for (int y = 0; y < TB; ++y) atomicAdd(&krows[(TA + y) * n + o4 + d], 2.0 * k24[y]);
+            for (int y = 0; y < TB; ++y) atomicAdd(&kd[TA + y], 2.0 * k24[y]);
         }
 #pragma unroll
-        for (int x = 0; x < TA; ++x) atomicAdd(&krows[x * n + o3 + c], 2.0 * k13[x]);
+        for (int x = 0; x < TA; ++x) atomicAdd(&kc[x], 2.0 * k13[x]);
 #pragma unroll
-        for (int y = 0; y < TB; ++y) atomicAdd(&krows[(TA + y) * n + o3 + c], 2.0 * k23[y]);
+        for (int y = 0; y < TB; ++y) atomicAdd(&kc[TA + y], 2.0 * k23[y]);
     }
-}
+};
 
 template <int LA, int LB, int LC, int LD, int TA, int TB>
-__device__ __forceinline__ void jk_tile_item(const JkTileArgs& a, int item, double* lds, int tile)
+__device__ __forceinline__ void jk_tile_item(const JkGroupArgs& g, const JkClassArgs& a, int item, double* lds, int tile)
 {
-    constexpr int N1 = (LA + 1) * (LA + 2) / 2, N2 = (LB + 1) * (LB + 2) / 2;
+    constexpr int N1 = (LA + 1) * (LA + 2) / 2, N2 = (LB + 1) * (LB + 2) / 2, N3 = (LC + 1) * (LC + 2) / 2;
     static_assert(N1 % TA == 0 && N2 % TB == 0, "tile must divide the bra components");
-    constexpr int NTB = N2 / TB, NR = TA + TB;
+    constexpr int NTB = N2 / TB, NR = TA + TB, RS = JkRows<TA, TB>::stride;
     const int a0 = (tile / NTB) * TA, b0 = (tile % NTB) * TB;
     const int tid = threadIdx.x, nt = blockDim.x;
     const JkItem it = a.items[item];
-    const MolInfo mi = a.mols[it.mol];
+    const MolInfo mi = g.mols[it.mol];
     const int n = mi.n;
-    double* drows = lds;            // NR rows of Dk: o1+a0.., then o2+b0..
-    double* krows = lds + NR * n;   // K' rows, same order
+    double* drows = lds;            // rows of Dk: o1+a0.., then o2+b0..
+    double* krows = lds + RS * n;   // K' rows, same order
     const int o1 = it.bra & 0x7fff, o2 = (it.bra >> 15) & 0x7fff;
     const double sbra = ((it.bra >> 30) & 1) ? 0.5 : 1.0;
-    const double* __restrict__ Dj = a.Dj + mi.base;
-    const double* __restrict__ Dk = a.Dk + mi.base;
-    double* const Jm = a.J + mi.base;
-    double* const Km = a.K + mi.base;
-    // stage the Dk rows eight elements a thread at a time, all eight loads
-    // issued before the first LDS write (the index is clamped into range so
-    // that no branch separates them; out-of-range slots are not written)
-    {
-        constexpr int SU = 8;
-        const int tot = NR * n;
-        for (int i0 = tid; i0 < tot; i0 += SU * nt) {
-            double v[SU];
+    const double* __restrict__ Dj = g.Dj + mi.base;
+    const double* __restrict__ Dk = g.Dk + mi.base;
+    double* const Jm = g.J + mi.base;
+    double* const Km = g.K + mi.base;
+    // the first unit's loads are in flight while the rows are staged
+    const int len = it.end - it.start, total = N3 * len;
+    JkUnit<LA, LB, LC, LD, TA, TB, double> un;
+    if (tid < total) un.load(a.l64, tid, it.start, len, n, Dj, a0, b0);
+    const double* __restrict__ ra = Dk + (size_t)(o1 + a0) * n;
+    const double* __restrict__ rb = Dk + (size_t)(o2 + b0) * n;
+    for (int c = tid; c < n; c += nt) {
+        double v[NR];
 #pragma unroll
-            for (int u = 0; u < SU; ++u) {
-                const int i = min(i0 + u * nt, tot - 1);
-                const int r = i / n, c = i - r * n;
-                const int row = r < TA ? o1 + a0 + r : o2 + b0 + (r - TA);
-                v[u] = Dk[(size_t)row * n + c];
-            }
+        for (int r = 0; r < NR; ++r) v[r] = r < TA ? ra[(size_t)r * n + c] : rb[(size_t)(r - TA) * n + c];
 #pragma unroll
-            for (int u = 0; u < SU; ++u) {
-                const int i = i0 + u * nt;
-                if (i < tot) {
-                    drows[i] = v[u];
-                    krows[i] = 0.0;
-                }
-            }
+        for (int r = 0; r < NR; ++r) {
+            drows[c * RS + r] = v[r];
+            krows[c * RS + r] = 0.0;
         }
     }
     double d12[TA][TB], j12[TA][TB];
@@ -414,22 +339,18 @@ __device__ __forceinline__ void jk_tile_item(const JkTileArgs& a, int item, doub
             j12[x][y] = 0.0;
         }
     __syncthreads();
-    if (JkRowSplit<LC, LD>::value) {
-        constexpr int N3 = (LC + 1) * (LC + 2) / 2;
-        jk_tile_rows<LA, LB, LC, LD, TA, TB, double>(a.l64, it.start, it.end, 0, drows, krows, n, Dj, sbra, d12, j12,
-                                                     a0, b0, tile);
-        if (a.items32) {
-            const int2 r32 = a.items32[item];
-            jk_tile_rows<LA, LB, LC, LD, TA, TB, float>(a.l32, r32.x, r32.y, N3 * (it.end - it.start), drows, krows,
-                                                        n, Dj, sbra, d12, j12, a0, b0, tile);
-        }
-    } else {
-        jk_tile_quartets<LA, LB, LC, LD, TA, TB, double>(a.l64, it.start, it.end, 0, drows, krows, n, Dj, sbra, d12,
-                                                         j12, a0, b0, tile);
-        if (a.items32) {
-            const int2 r32 = a.items32[item];
-            jk_tile_quartets<LA, LB, LC, LD, TA, TB, float>(a.l32, r32.x, r32.y, it.end - it.start, drows, krows, n,
-                                                            Dj, sbra, d12, j12, a0, b0, tile);
+    for (int u = tid; u < total;) {
+        un.digest(a.l64, drows, krows, sbra, d12, j12, tile);
+        u += nt;
+        if (u < total) un.load(a.l64, u, it.start, len, n, Dj, a0, b0);
+    }
+    if (a.items32) {
+        const int2 r32 = a.items32[item];
+        const int len32 = r32.y - r32.x, total32 = N3 * len32;
+        JkUnit<LA, LB, LC, LD, TA, TB, float> uf;
+        for (int u = (tid - total % nt + nt) % nt; u < total32; u += nt) {
+            uf.load(a.l32, u, r32.x, len32, n, Dj, a0, b0);
+            uf.digest(a.l32, drows, krows, sbra, d12, j12, tile);
         }
     }
 #pragma unroll
@@ -440,23 +361,41 @@ __device__ __forceinline__ void jk_tile_item(const JkTileArgs& a, int item, doub
             if ((tid & 63) == 0 && s != 0.0) atomic_addd(&Jm[(size_t)(o1 + a0 + x) * n + o2 + b0 + y], s);
         }
     __syncthreads();
-    for (int i = tid; i < NR * n; i += nt) {
-        const double v = krows[i];
-        if (v != 0.0) {
-            const int r = i / n, c = i - r * n;
-            const int row = r < TA ? o1 + a0 + r : o2 + b0 + (r - TA);
-            atomic_addd(&Km[(size_t)row * n + c], v);
-        }
+    double* const ka = Km + (size_t)(o1 + a0) * n;
+    double* const kb = Km + (size_t)(o2 + b0) * n;
+    for (int c = tid; c < n; c += nt) {
+        double v[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) v[r] = krows[c * RS + r];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+            if (v[r] != 0.0) atomic_addd(r < TA ? &ka[(size_t)r * n + c] : &kb[(size_t)(r - TA) * n + c], v[r]);
     }
     __syncthreads();
 }
 
+// block `local` of a class: bra tile local / grid, items local % grid, + grid, ...
 template <int LA, int LB, int LC, int LD, int TA, int TB>
-__global__ void __launch_bounds__(256) jk_tile_kernel(const JkTileArgs a)
+__device__ __forceinline__ void jk_tile_class(const JkGroupArgs& g, const JkClassArgs& a, int local, double* lds)
 {
-    extern __shared__ double lds[];
-    for (int item = blockIdx.x; item < a.nitems; item += gridDim.x)
-        jk_tile_item<LA, LB, LC, LD, TA, TB>(a, item, lds, blockIdx.y);
+    const int tile = local / a.grid;
+    for (int item = local - tile * a.grid; item < a.nitems; item += a.grid)
+        jk_tile_item<LA, LB, LC, LD, TA, TB>(g, a, item, lds, tile);
+}
+
+__device__ __forceinline__ int jk_group_slot(const JkGroupArgs& g)
+{
+    int s = 0;
+    while (s + 1 < g.n && (int)blockIdx.x >= g.c[s + 1].block0) ++s;
+    return s;
+}
+
+__device__ __forceinline__ void jk_clock(const JkGroupArgs& g, int cls, int end)
+{
+    if (!g.clock || threadIdx.x) return;
+    const unsigned long long t = wall_clock64();
+    if (end) atomicMax(&g.clock[2 * cls + 1], t);
+    else atomicMin(&g.clock[2 * cls], t);
 }
 
 // Dense scatter with 8-fold permutational symmetry (Methods/hartree_fock.py:314-325)

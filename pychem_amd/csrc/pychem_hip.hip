@@ -446,18 +446,15 @@ struct pq_basis {
     int ev_jk_used = 0;
     hipEvent_t ev_pass[2] = {};   // whole ERI pass on the caller's stream
     int ev_pass_used = 0;
-    // per-class J/K digestion launches (timing on): events around each
-    // class's kernel on the stream it ran on, summed over calls
-    hipEvent_t ev_jkc[ERI_NCLASS][2] = {};
-    int jkc_pending[ERI_NCLASS] = {};
-    double jkc_sum[ERI_NCLASS] = {};
-    long long jkc_n[ERI_NCLASS] = {};
+    // per-class J/K digestion times (timing on), on the device: per class the
+    // current call's first block start and last block end, then the sum of
+    // the spans and the number of calls, in ticks of the realtime clock
+    DevBuf d_jkclock;
     hipGraphExec_t graph_exec = nullptr;
     // Class launches fan out over side streams (default priority); with the
     // caller's stream, four streams fill the process's four hardware queues.
-    // J/K: jk_nstreams streams, the caller's one of them (C20H42 J/K alone
-    // 1.32 / 1.33 / 1.28 ms on 2 / 3 / 4; with every stream a side stream,
-    // 4 had been slower than 3).  Schwarz and ERI passes: eri_nstreams side
+    // J/K: jk_nstreams streams, the caller's one of them (C20H42: 1.24 ms on
+    // one, 1.21 on four).  Schwarz and ERI passes: eri_nstreams side
     // streams beside the caller's, which runs the fused heavy classes.
     int jk_nstreams = 4;
     int eri_nstreams = 3;
@@ -502,24 +499,29 @@ static int ensure_events(pq_basis* b)
     HIPCHK(hipEventCreate(&b->ev_jk[1]));
     HIPCHK(hipEventCreate(&b->ev_pass[0]));
     HIPCHK(hipEventCreate(&b->ev_pass[1]));
-    for (int c = 0; c < ERI_NCLASS; ++c)
-        for (int k = 0; k < 2; ++k) HIPCHK(hipEventCreate(&b->ev_jkc[c][k]));
     return 0;
 }
 
-// Add the finished per-class J/K timings of earlier calls to the sums.
-static int collect_jk_class_times(pq_basis* b)
+// Per class: the call's span (set = 0: empty it; 1: add it to the sums; 2:
+// clear everything).
+__global__ void jk_clock_kernel(unsigned long long* clock, int set)
 {
-    for (int c = 0; c < ERI_NCLASS; ++c) {
-        if (!b->jkc_pending[c]) continue;
-        HIPCHK(hipEventSynchronize(b->ev_jkc[c][1]));
-        float ms = 0.f;
-        HIPCHK(hipEventElapsedTime(&ms, b->ev_jkc[c][0], b->ev_jkc[c][1]));
-        b->jkc_sum[c] += ms;
-        b->jkc_n[c] += 1;
-        b->jkc_pending[c] = 0;
+    const int c = threadIdx.x;
+    if (c >= ERI_NCLASS) return;
+    unsigned long long* sum = clock + 2 * ERI_NCLASS;
+    if (set == 2) sum[2 * c] = sum[2 * c + 1] = 0;
+    if (set == 1 && clock[2 * c + 1] > clock[2 * c]) {
+        sum[2 * c] += clock[2 * c + 1] - clock[2 * c];
+        sum[2 * c + 1] += 1;
     }
-    return 0;
+    clock[2 * c] = ~0ULL;
+    clock[2 * c + 1] = 0;
+}
+
+static void jk_clock_set(pq_basis* b, int set, hipStream_t st)
+{
+    if (b->timing && b->d_jkclock.p)
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, st, (unsigned long long*)b->d_jkclock.p, set);
 }
 
 extern "C" const char* pq_last_error(void) { return g_err.c_str(); }
@@ -850,8 +852,6 @@ extern "C" void pq_basis_destroy(pq_basis* b)
         (void)hipEventDestroy(b->ev_jk[1]);
         (void)hipEventDestroy(b->ev_pass[0]);
         (void)hipEventDestroy(b->ev_pass[1]);
-        for (int c = 0; c < ERI_NCLASS; ++c)
-            for (int k = 0; k < 2; ++k) (void)hipEventDestroy(b->ev_jkc[c][k]);
     }
     if (b->ev_fork) {
         for (int k = 0; k < 4; ++k) {
@@ -1285,11 +1285,6 @@ static inline bool jk_tile_fits(const pq_basis* b, int cls)
     return b->nmax < 32768 && sizeof(double) * (size_t)jk_tile_table[cls][3] * b->nmax <= 65536;
 }
 
-static inline int jk_grid_of(const EriClassStore& s)
-{
-    return (s.jk_grid > 0 && s.jk_grid < s.nitems) ? s.jk_grid : s.nitems;
-}
-
 // The two-electron operator of the class kernels (Methods/_c_ints.c:236-239
 // dispatches on ints_type): 0 the Coulomb operator, 1 the electron-scattering
 // operator at momentum transfer grid_value (Methods/c_ints/
@@ -1686,20 +1681,31 @@ extern "C" int pq_eri_build(pq_basis* b, double threshold, double fp32_threshold
 extern "C" int pq_eri_recompute(pq_basis* b, void* stream) { return pq_eri_compute(b, stream); }
 
 // Per-class J/K digestion times summed over the calls made with timing on
-// (pq_jk, pq_jk_general, the J/K of pq_scf_run), launch counts and the
-// classes' work items; reset != 0 clears the sums afterwards.
+// (pq_jk, pq_jk_general, the J/K of pq_scf_run): from the start of a class's
+// first block to the end of its last, by the GPU's realtime clock (the classes
+// of a call share launches); calls counted and the classes' work items; reset
+// != 0 clears the sums afterwards.  Waits for the device.
 extern "C" int pq_jk_class_times(pq_basis* b, double* sum_ms, long long* launches, long long* nitems, int reset)
 {
     if (!b) return fail("pq_jk_class_times: null basis");
-    if (b->timing && collect_jk_class_times(b)) return -1;
+    unsigned long long h[2 * ERI_NCLASS] = {};
+    double ms_per_tick = 0.0;
+    if (b->d_jkclock.p) {
+        int dev = 0, khz = 0;
+        HIPCHK(hipGetDevice(&dev));
+        HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+        if (khz > 0) ms_per_tick = 1.0 / khz;
+        HIPCHK(hipDeviceSynchronize());
+        HIPCHK(hipMemcpy(h, (unsigned long long*)b->d_jkclock.p + 2 * ERI_NCLASS, sizeof(h), hipMemcpyDeviceToHost));
+    }
     for (int c = 0; c < ERI_NCLASS; ++c) {
-        if (sum_ms) sum_ms[c] = b->jkc_sum[c];
-        if (launches) launches[c] = b->jkc_n[c];
+        if (sum_ms) sum_ms[c] = (double)h[2 * c] * ms_per_tick;
+        if (launches) launches[c] = (long long)h[2 * c + 1];
         if (nitems) nitems[c] = b->store64[c].nitems;
-        if (reset) {
-            b->jkc_sum[c] = 0.0;
-            b->jkc_n[c] = 0;
-        }
+    }
+    if (reset && b->d_jkclock.p) {
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
+        HIPCHK(hipDeviceSynchronize());
     }
     return 0;
 }
@@ -1708,7 +1714,13 @@ extern "C" int pq_set_timing(pq_basis* b, int on)
 {
     if (!b) return fail("pq_set_timing: null basis");
     b->timing = on ? 1 : 0;
-    if (b->timing) return ensure_events(b);
+    if (!b->timing) return 0;
+    if (ensure_events(b)) return -1;
+    if (!b->d_jkclock.p) {
+        if (b->d_jkclock.ensure(sizeof(unsigned long long) * 4 * ERI_NCLASS)) return -1;
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
+        HIPCHK(hipDeviceSynchronize());
+    }
     return 0;
 }
 
@@ -1787,61 +1799,107 @@ extern "C" int pq_eri_nclass(void) { return ERI_NCLASS; }
 // One class into J', K'.  part: 1 = tiled digestion kernel, 2 = ket J
 // reductions, 3 = both.  lists: bit 0 the FP64 list, bit 1 the FP32 list; the
 // tiled kernel digests both in one launch.
+// One class's entry of a group launch (lists: 1 FP64, 2 FP32, 3 both).
+// Returns its blocks; 0 when it has nothing to digest.
+static int jk_class_args(pq_basis* b, int c, int lists, JkClassArgs& a)
+{
+    const EriClassStore& s64 = b->store64[c];
+    const EriClassStore& s32 = b->store32[c];
+    const bool u64 = (lists & 1) && s64.nq, u32 = (lists & 2) && s32.nq;
+    if ((!u64 && !u32) || s64.nitems <= 0) return 0;
+    a.items = (const JkItem*)s64.items.p;
+    a.items32 = u32 ? (const int2*)s64.items32.p : (const int2*)nullptr;
+    a.l64 = JkTileList<double>{(const unsigned*)s64.kets.p, (const double*)s64.vals.p, (double*)s64.jkbuf.p, s64.nq};
+    a.l32 = JkTileList<float>{(const unsigned*)s32.kets.p, (const float*)s32.vals.p, (double*)s32.jkbuf.p, s32.nq};
+    a.nitems = s64.nitems;
+    const int tuned = s64.jk_grid > 0 ? s64.jk_grid : s32.jk_grid;
+    a.grid = (tuned > 0 && tuned < a.nitems) ? tuned : a.nitems;
+    a.cls = c;
+    return a.grid * jk_tile_table[c][2];
+}
+
+// Work units of a class (quartets, or (quartet, ket row) pairs where the
+// kernel splits the rows).
+static double jk_class_units(const pq_basis* b, int c, int lists)
+{
+    const int n3 = ncart_l(eri_class_table[c][2]), n4 = ncart_l(eri_class_table[c][3]);
+    const double units = (n3 * n4 >= 3) ? (double)n3 : 1.0;
+    return units * (double)(((lists & 1) ? b->store64[c].nq : 0) + ((lists & 2) ? b->store32[c].nq : 0));
+}
+
+// The listed classes in one launch of group kernel `group`: threads per block
+// from the mean work units per item.
+static int jk_group_launch(pq_basis* b, int group, const int* classes, int nc, int lists, const double* Dj,
+                           const double* Dk, double* J, double* K, hipStream_t st)
+{
+    JkGroupArgs g;
+    g.n = 0;
+    long long blocks = 0;
+    double units = 0.0, items = 0.0;
+    size_t rows = 0;
+    for (int k = 0; k < nc; ++k) {
+        const int c = classes[k];
+        JkClassArgs& a = g.c[g.n];
+        const int nb = jk_class_args(b, c, lists, a);
+        if (!nb) continue;
+        a.block0 = (int)blocks;
+        blocks += nb;
+        if (blocks > 0x7fffffffLL) return fail("J/K digestion grid too large");
+        units += jk_class_units(b, c, lists);
+        items += a.nitems;
+        rows = std::max(rows, (size_t)jk_tile_table[c][3]);
+        ++g.n;
+    }
+    if (!g.n) return 0;
+    g.mols = (const MolInfo*)b->d_mols.p;
+    g.Dj = Dj;
+    g.Dk = Dk;
+    g.J = J;
+    g.K = K;
+    g.clock = b->timing ? (unsigned long long*)b->d_jkclock.p : nullptr;
+    const double mean = units / std::max(1.0, items);
+    const int block = mean > 160.0 ? 256 : (mean > 80.0 ? 128 : 64);
+    jk_group_run[group](g, (int)blocks, block, sizeof(double) * rows * b->nmax, st);
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+// A class too wide for the tiled kernels' LDS rows, one thread per quartet.
+static int jk_launch_untiled(pq_basis* b, int c, const double* Dj, const double* Dk, double* J, double* K,
+                             hipStream_t st, int lists)
+{
+    const EriClassStore& s64 = b->store64[c];
+    const EriClassStore& s32 = b->store32[c];
+    const MolInfo* dm = (const MolInfo*)b->d_mols.p;
+    if ((lists & 1) && s64.nq) {
+        JkArgs<double> a{(const int2*)s64.q.p, (const PairHdr*)b->d_pairs.p, (const int*)b->d_cart_off.p, dm,
+                         (const double*)s64.vals.p, Dj, Dk, J, K, s64.nq, b->nmax};
+        jk_launch<double>(c, a, st);
+    }
+    if ((lists & 2) && s32.nq) {
+        JkArgs<float> a{(const int2*)s32.q.p, (const PairHdr*)b->d_pairs.p, (const int*)b->d_cart_off.p, dm,
+                        (const float*)s32.vals.p, Dj, Dk, J, K, s32.nq, b->nmax};
+        jk_launch<float>(c, a, st);
+    }
+    HIPCHK(hipGetLastError());
+    return 0;
+}
+
+// One class alone: part 1 the digestion, 2 the ket J reduction of its tiled
+// lists, 3 both.
 static int jk_launch_class(pq_basis* b, int c, const double* Dj, const double* Dk, double* J, double* K,
                            hipStream_t st, int part = 3, int lists = 3)
 {
-    EriClassStore& s64 = b->store64[c];
-    EriClassStore& s32 = b->store32[c];
-    const bool u64 = (lists & 1) && s64.nq, u32 = (lists & 2) && s32.nq;
-    if (!u64 && !u32) return 0;
-    const MolInfo* dm = (const MolInfo*)b->d_mols.p;
-    if (jk_tile_fits(b, c)) {
-        if (part & 1) {
-            JkTileArgs a;
-            a.items = (const JkItem*)s64.items.p;
-            a.items32 = u32 ? (const int2*)s64.items32.p : (const int2*)nullptr;
-            a.l64 = JkTileList<double>{(const unsigned*)s64.kets.p, (const double*)s64.vals.p, (double*)s64.jkbuf.p,
-                                       s64.nq};
-            a.l32 = JkTileList<float>{(const unsigned*)s32.kets.p, (const float*)s32.vals.p, (double*)s32.jkbuf.p,
-                                      s32.nq};
-            a.mols = dm;
-            a.Dj = Dj;
-            a.Dk = Dk;
-            a.J = J;
-            a.K = K;
-            a.nmax = b->nmax;
-            const int items = s64.nitems;
-            a.nitems = items;
-            const int tuned = s64.jk_grid > 0 ? s64.jk_grid : s32.jk_grid;
-            a.grid = (tuned > 0 && tuned < items) ? tuned : items;
-            // threads per block from the mean work units per item: quartets,
-            // or (quartet, ket row) pairs where the kernel splits the rows
-            const int n3 = ncart_l(eri_class_table[c][2]), n4 = ncart_l(eri_class_table[c][3]);
-            const double units = (n3 * n4 >= 3) ? (double)n3 : 1.0;
-            const double mean = units * (double)((u64 ? s64.nq : 0) + (u32 ? s32.nq : 0)) / std::max(1, items);
-            const int block = mean > 160.0 ? 256 : (mean > 80.0 ? 128 : 64);
-            if (items > 0) jktile_launch(c, a, block, st);
-        }
-        if (part & 2) {
-            const int n3 = ncart_l(eri_class_table[c][2]), n4 = ncart_l(eri_class_table[c][3]);
-            for (int w = 0; w < 2; ++w) {
-                EriClassStore& s = w ? s32 : s64;
-                if (!(w ? u32 : u64)) continue;
-                jket_reduce(jred_list(list_args(b, c), list_bras(s), w, (const double*)s.jkbuf.p, s.nq,
-                                      jk_tile_table[c][2], n3 * n4, n4, s.jtiles, s.njtile),
-                            dm, J, st);
-            }
-        }
-    } else {
-        if (u64) {
-            JkArgs<double> a{(const int2*)s64.q.p, (const PairHdr*)b->d_pairs.p, (const int*)b->d_cart_off.p, dm,
-                             (const double*)s64.vals.p, Dj, Dk, J, K, s64.nq, b->nmax};
-            jk_launch<double>(c, a, st);
-        }
-        if (u32) {
-            JkArgs<float> a{(const int2*)s32.q.p, (const PairHdr*)b->d_pairs.p, (const int*)b->d_cart_off.p, dm,
-                            (const float*)s32.vals.p, Dj, Dk, J, K, s32.nq, b->nmax};
-            jk_launch<float>(c, a, st);
+    if (!jk_tile_fits(b, c)) return jk_launch_untiled(b, c, Dj, Dk, J, K, st, lists);
+    if ((part & 1) && jk_group_launch(b, jk_group_table[c], &c, 1, lists, Dj, Dk, J, K, st)) return -1;
+    if (part & 2) {
+        const int n3 = ncart_l(eri_class_table[c][2]), n4 = ncart_l(eri_class_table[c][3]);
+        for (int w = 0; w < 2; ++w) {
+            EriClassStore& s = w ? b->store32[c] : b->store64[c];
+            if (!((lists >> w) & 1) || !s.nq) continue;
+            jket_reduce(jred_list(list_args(b, c), list_bras(s), w, (const double*)s.jkbuf.p, s.nq,
+                                  jk_tile_table[c][2], n3 * n4, n4, s.jtiles, s.njtile),
+                        (const MolInfo*)b->d_mols.p, J, st);
         }
     }
     HIPCHK(hipGetLastError());
@@ -1849,54 +1907,86 @@ static int jk_launch_class(pq_basis* b, int c, const double* Dj, const double* D
 }
 
 // Zero J', K'; digest every stored class; add the ket J values of all tiled
-// lists in one reduction launch; symmetrise.  With jk_nstreams > 1 the class
-// launches fork from `st` onto side streams (largest stored bytes first, each
-// to the least-loaded stream) and join back before the reduction, so that
-// small high-l classes overlap the large ones.  (Each class's reduction
-// launched behind its digestion on the side stream instead was slower: the
-// many small reduction launches queue behind the digestion kernels.)
-static int jk_digest_all(pq_basis* b, const double* Dj, const double* Dk, double* J, double* K, hipStream_t st)
+// lists in one reduction launch; symmetrise.  The classes go in one launch per
+// register / LDS group (jk_group_table; one launch per class, 21 of them, was
+// bound by the host: C10H22 387 us, CH3OH 152 us per build; one kernel over
+// every class spilled 2.4 KB a lane), the groups over jk_nstreams streams:
+// forked from `st` onto side streams (most stored bytes first, each
+// to the least-loaded stream) and joined back before the reduction.  (Each
+// class's reduction launched behind its digestion on the side stream instead
+// was slower: the many small reduction launches queue behind the digestion
+// kernels.)
+static int jk_digest_all(pq_basis* b, const double* Dj, const double* Dk, double* J, double* K, hipStream_t st,
+                         bool single_stream)
 {
-    std::vector<std::pair<double, int>> order;
+    // classes by stored bytes per block, so that the longest blocks start first
+    int order[ERI_NCLASS], nc = 0;
+    double bytes[ERI_NCLASS] = {}, per[ERI_NCLASS] = {};
+    long long blocks = 0;
+    bool untiled = false;
     for (int c = 0; c < ERI_NCLASS; ++c) {
-        double bytes = 0.0;
         for (int w = 0; w < 2; ++w) {
             const EriClassStore& s = w ? b->store32[c] : b->store64[c];
-            bytes += (double)s.nq * s.ncomp * (w ? 4.0 : 8.0) + 16.0 * s.nq;
+            bytes[c] += (double)s.nq * s.ncomp * (w ? 4.0 : 8.0) + 16.0 * s.nq;
         }
-        if (bytes > 0.0) order.push_back({bytes, c});
+        if (!(bytes[c] > 0.0)) continue;
+        if (!jk_tile_fits(b, c)) {
+            untiled = true;
+            continue;
+        }
+        JkClassArgs a;
+        const int nb = jk_class_args(b, c, 3, a);
+        per[c] = bytes[c] / std::max(1, nb);
+        blocks += nb;
+        int k = nc++;
+        for (; k > 0 && per[order[k - 1]] < per[c]; --k) order[k] = order[k - 1];
+        order[k] = c;
     }
-    std::sort(order.begin(), order.end(), [](const std::pair<double, int>& u, const std::pair<double, int>& v) {
-        return u.first > v.first;
-    });
-    // the caller's stream is one of the ns streams (its first class starts
-    // behind the zero fill with no cross-stream wait), side streams the rest
-    const int ns = std::min(4, std::max(1, b->jk_nstreams));
+    jk_clock_set(b, 0, st);
+    if (untiled)
+        for (int c = 0; c < ERI_NCLASS; ++c)
+            if (bytes[c] > 0.0 && !jk_tile_fits(b, c) && jk_launch_untiled(b, c, Dj, Dk, J, K, st, 3)) return -1;
+    int in[JK_NGROUP][ERI_NCLASS], ng[JK_NGROUP] = {};
+    double gb[JK_NGROUP] = {};
+    int gorder[JK_NGROUP], n = 0;
+    for (int k = 0; k < nc; ++k) {
+        const int c = order[k], g = jk_group_table[c];
+        in[g][ng[g]++] = c;
+        gb[g] += bytes[c];
+    }
+    for (int g = 0; g < JK_NGROUP; ++g) {
+        if (!ng[g]) continue;
+        int k = n++;
+        for (; k > 0 && gb[gorder[k - 1]] < gb[g]; --k) gorder[k] = gorder[k - 1];
+        gorder[k] = g;
+    }
+    // The caller's stream is one of the ns streams (its first group starts
+    // behind the zero fill with no cross-stream wait), side streams the rest.
+    // Below 400 MB of stored integrals every group goes on the caller's
+    // stream: the fork and join cost more than the overlap of the groups'
+    // ends gains (CH3OH 99 us on four streams, 52 on one; C7H15OH, 150 MB, two
+    // digestions, 458 / 441; C10H22, 0.55 GB, 309 / 315; C14H30 613 / 654).
+    const bool small = gb[0] + gb[1] + gb[2] + gb[3] < 400e6;
+    const int ns = single_stream || small ? 1 : std::min(n, std::min(4, std::max(1, b->jk_nstreams)));
     if (ns > 1) {
         if (ensure_jk_streams(b)) return -1;
         HIPCHK(hipEventRecord(b->ev_fork, st));
         for (int k = 1; k < ns; ++k) HIPCHK(hipStreamWaitEvent(b->jk_side[k - 1], b->ev_fork, 0));
     }
-    if (b->timing && collect_jk_class_times(b)) return -1;
     double load[4] = {0.0, 0.0, 0.0, 0.0};
-    for (const auto& o : order) {
+    for (int q = 0; q < n; ++q) {
+        const int g = gorder[q];
         int k = 0;
         for (int t = 1; t < ns; ++t)
             if (load[t] < load[k]) k = t;
-        load[k] += o.first;
-        hipStream_t sk = k > 0 ? b->jk_side[k - 1] : st;
-        if (b->timing) HIPCHK(hipEventRecord(b->ev_jkc[o.second][0], sk));
-        if (jk_launch_class(b, o.second, Dj, Dk, J, K, sk, 1)) return -1;
-        if (b->timing) {
-            HIPCHK(hipEventRecord(b->ev_jkc[o.second][1], sk));
-            b->jkc_pending[o.second] = 1;
-        }
+        load[k] += gb[g];
+        if (jk_group_launch(b, g, in[g], ng[g], 3, Dj, Dk, J, K, k > 0 ? b->jk_side[k - 1] : st)) return -1;
     }
-    if (ns > 1)
-        for (int k = 1; k < ns; ++k) {
-            HIPCHK(hipEventRecord(b->ev_join[k - 1], b->jk_side[k - 1]));
-            HIPCHK(hipStreamWaitEvent(st, b->ev_join[k - 1], 0));
-        }
+    for (int k = 1; k < ns; ++k) {
+        HIPCHK(hipEventRecord(b->ev_join[k - 1], b->jk_side[k - 1]));
+        HIPCHK(hipStreamWaitEvent(st, b->ev_join[k - 1], 0));
+    }
+    jk_clock_set(b, 1, st);
     return 0;
 }
 
@@ -1912,7 +2002,7 @@ static int jk_launch_all(pq_basis* b, const double* Dj, const double* Dk, double
 {
     const MolInfo* dm = (const MolInfo*)b->d_mols.p;
     jk_zero(b, J, K, st);
-    if (jk_digest_all(b, Dj, Dk, J, K, st)) return -1;
+    if (jk_digest_all(b, Dj, Dk, J, K, st, false)) return -1;
     jket_reduce_all((const JredList*)b->d_jred.p, b->njred, b->jred_blocks, dm, J, st);
     int gx = (int)((b->nmax * (long long)b->nmax + 255) / 256);
     gx = gx < 1 ? 1 : (gx > 64 ? 64 : gx);
@@ -2001,12 +2091,7 @@ static int jk_general_run(pq_basis* b, const double* Dj, const double* Dk, doubl
         double* Kp = pass ? K : K2;
         const double* Dkp = pass ? (const double*)DkT : Dk;
         jk_zero(b, Jp, Kp, st);
-        if (single_stream) {
-            for (int c = 0; c < ERI_NCLASS; ++c)
-                if (jk_launch_class(b, c, Ds, Dkp, Jp, Kp, st, 1)) return -1;
-        } else if (jk_digest_all(b, Ds, Dkp, Jp, Kp, st)) {
-            return -1;
-        }
+        if (jk_digest_all(b, Ds, Dkp, Jp, Kp, st, single_stream)) return -1;
     }
     jket_reduce_all((const JredList*)b->d_jred.p, b->njred, b->jred_blocks, dm, J, st);
     hipLaunchKernelGGL(jk_general_finish_kernel, dim3(gx, b->nmol), dim3(256), 0, st, J, K, K2, dm);

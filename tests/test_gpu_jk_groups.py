@@ -1,0 +1,83 @@
+"""The grouped J/K launches: molecules of one atom and one class upward, FP32
+lists, one stream and four, persistent blocks, the timed build and the
+allocation-free entry against a float64 contraction of the dense integrals.
+
+Tolerance: each matrix element sums at most n^2 products, rounded once per
+addition; FP32 lists hold values rounded to 2^-24 of themselves, which the
+dense tensor holds as well.
+"""
+import numpy as np
+import pytest
+
+from pychem_amd import geometry, structures
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -53
+
+
+def _case(rows, basis, cartesian, fp32, seed):
+    import torch
+    from pychem_amd.engine import Engine
+    m = structures.Molecule(rows, basis=basis, cartesian_l=cartesian, multiplicity=1)
+    e = Engine(m)
+    e.build_eri(1e-8, fp32)
+    n = e.ncart
+    rng = np.random.default_rng(seed)
+    D = rng.normal(size=(2, n, n))
+    D = D + D.transpose(0, 2, 1)
+    t = torch.empty((n, n, n, n), dtype=torch.float64, device="cuda")
+    from pychem_amd import _lib
+    from pychem_amd.engine import _ptr, _stream
+    _lib.check(_lib.lib().pq_eri_dense(e.h, _ptr(t), _stream()), "pq_eri_dense")
+    eri = t.cpu().numpy()
+    J = np.einsum("abcd,cd->ab", eri, D[0], optimize=True)
+    K = -np.einsum("abcd,cb->ad", eri, D[1], optimize=True)
+    Jm = np.einsum("abcd,cd->ab", np.abs(eri), np.abs(D[0]), optimize=True)
+    Km = np.einsum("abcd,cb->ad", np.abs(eri), np.abs(D[1]), optimize=True)
+    tol = 4 * (n * n + 16) * U
+    return e, torch.as_tensor(D, device="cuda"), (J, tol * Jm), (K, tol * Km)
+
+
+def _jk(e, D, fn="pq_jk"):
+    import torch
+    from pychem_amd import _lib
+    from pychem_amd.engine import _ptr, _stream
+    J, K = torch.full_like(D[0], 7.0), torch.full_like(D[0], 7.0)
+    _lib.check(getattr(_lib.lib(), fn)(e.h, _ptr(D[0]), _ptr(D[1]), _ptr(J), _ptr(K), _stream()), fn)
+    return J.cpu().numpy(), K.cpu().numpy()
+
+
+ROWS = {"He": [["He", 2.0, 0.0, 0.0, 0.0]], "Ne": [["Ne", 10.0, 0.0, 0.0, 0.0]],
+        "H2O": geometry.small_molecule("H2O", 0.05, 3), "CH3OH": geometry.small_molecule("CH3OH", 0.05, 4),
+        "C4H10": geometry.alkane(4, 0.05, 5)}
+
+
+@pytest.mark.parametrize("name,basis,cartesian,fp32", [
+    ("He", "STO-3G", [2], 0.0), ("He", "6-31G*", [2], 0.0), ("Ne", "6-31G*", [2], 0.0), ("H2O", "STO-3G", [2], 1e-3),
+    ("CH3OH", "6-31G*", [2], 0.0), ("CH3OH", "6-31G*", [2], 1e-2), ("C4H10", "6-31G*", [2], 1e-5),
+    ("C4H10", "6-311G*", [2], 0.0)])
+def test_builds_against_the_dense_integrals(gpu, name, basis, cartesian, fp32):
+    from pychem_amd import _lib
+    L = _lib.lib()
+    e, D, (J, eJ), (K, eK) = _case(ROWS[name], basis, cartesian, fp32, len(name))
+
+    def check(got):
+        assert (np.abs(got[0] - J) <= eJ).all() and (np.abs(got[1] - K) <= eK).all()
+
+    for ns in (1, 4):
+        _lib.check(L.pq_jk_set_streams(e.h, ns), "pq_jk_set_streams")
+        check(_jk(e, D))
+    check(_jk(e, D, "pq_jk_general"))
+    check(_jk(e, D, "pq_jk_general_noalloc"))
+    for cls in range(L.pq_eri_nclass()):          # short items, three persistent blocks a tile
+        _lib.check(L.pq_jk_set_params(e.h, cls, 64, 3, None), "pq_jk_set_params")
+    check(_jk(e, D))
+    e.set_timing(True)
+    e.jk_class_times(reset=True)
+    check(_jk(e, D))
+    check(_jk(e, D))
+    ms, calls, items = e.jk_class_times()
+    stored = np.array([s["nq64"] + s["nq32"] > 0 for s in e.stats()])
+    assert (calls[stored] == 2).all() and (calls[~stored] == 0).all()
+    assert (ms[stored] > 0.0).all() and (ms < 100.0).all() and (items[stored] > 0).all()
+    e.close()
