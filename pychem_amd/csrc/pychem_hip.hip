@@ -1279,10 +1279,12 @@ static int build_items(pq_basis* b, int c, hipStream_t st)
 }
 
 // The tiled kernel packs offsets into 15 bits and keeps 2 (TA + TB) rows of
-// the largest molecule in LDS (at most 64 KiB).
+// the largest molecule in LDS, all 160 KiB of a CU if need be: C30H62 (n = 574,
+// 83 KB for the nine-row tiles) 3.06 ms per build, 10.9 ms when those classes
+// went one thread per quartet from 64 KiB on.
 static inline bool jk_tile_fits(const pq_basis* b, int cls)
 {
-    return b->nmax < 32768 && sizeof(double) * (size_t)jk_tile_table[cls][3] * b->nmax <= 65536;
+    return b->nmax < 32768 && sizeof(double) * (size_t)jk_tile_table[cls][3] * b->nmax <= 163840;
 }
 
 // The two-electron operator of the class kernels (Methods/_c_ints.c:236-239

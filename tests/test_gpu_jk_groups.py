@@ -81,3 +81,37 @@ def test_builds_against_the_dense_integrals(gpu, name, basis, cartesian, fp32):
     assert (calls[stored] == 2).all() and (calls[~stored] == 0).all()
     assert (ms[stored] > 0.0).all() and (ms < 100.0).all() and (items[stored] > 0).all()
     e.close()
+
+
+def test_rows_beyond_64_kib_of_lds(gpu):
+    """Three distant octanes in one molecule (468 functions: 67 KB of rows for
+    the nine-row tiles): with a density on one of them its own J block, and
+    every octane's K block, are those of the octane alone, to the rounding of
+    the same sums in another order."""
+    import torch
+    from pychem_amd.engine import Engine
+    one = geometry.alkane(8, 0.02, 9)
+    far = [[r[0], r[1], r[2], r[3] + 200.0 * k, r[4]] for k in range(3) for r in one]
+    ms = [structures.Molecule(rows, basis="6-31G*", cartesian_l=[2]) for rows in (one, far)]
+    es = [Engine(m) for m in ms]
+    for e in es:
+        e.build_eri(1e-8)
+    n = es[0].ncart
+    assert es[1].ncart == 3 * n and 9 * 16 * 3 * n > 65536
+    # fragments of the long molecule hold the same atoms in the same order
+    rng = np.random.default_rng(8)
+    A = rng.normal(size=(n, n))
+    D = torch.as_tensor(A + A.T, device="cuda")
+    J1, K1 = es[0].jk(D, D)
+    Dj, Dk = (torch.zeros((3 * n, 3 * n), dtype=torch.float64, device="cuda") for _ in range(2))
+    Dj[:n, :n] = D
+    for k in range(3):
+        Dk[k * n:(k + 1) * n, k * n:(k + 1) * n] = D
+    J3, K3 = es[1].jk(Dj, Dk)
+    # translations round the coordinates of two of them (200 A: 2^-53 * 400 bohr)
+    assert (J3[:n, :n] - J1).abs().max().item() < 1e-11 * J1.abs().max().item()
+    for k in range(3):
+        blk = K3[k * n:(k + 1) * n, k * n:(k + 1) * n]
+        assert (blk - K1).abs().max().item() < 1e-10 * K1.abs().max().item()
+    for e in es:
+        e.close()
