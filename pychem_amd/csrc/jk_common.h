@@ -22,6 +22,51 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// Sums of T per-lane values over the wave: value 4 u + {0, 2, 1, 3}[lane / 16]
+// ends in out[u] of that row's lanes.  The first two halvings swap halves and
+// rows between two values, so that each swap and addition serves both; within a
+// row of 16 lanes the values rotate (DPP).  No LDS: a shuffle per step and
+// value was a third of the digestion's LDS instructions (18 values: 216 of
+// them, against 102 vector instructions here).
+__device__ __forceinline__ double swap_add32(double a, double b)
+{
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+__device__ __forceinline__ double swap_add16(double a, double b)
+{
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
+template <int CTRL>
+__device__ __forceinline__ double rotate_add(double a)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, 0xf, 0xf, false);
+    return a + __hiloint2double(hi, lo);
+}
+
+template <int T>
+__device__ __forceinline__ void wave_sums(const double (&v)[T], double (&out)[(T + 3) / 4])
+{
+    constexpr int H = (T + 1) / 2, U = (T + 3) / 4;
+    double h[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) h[i] = swap_add32(v[2 * i], 2 * i + 1 < T ? v[2 * i + 1] : 0.0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        double s = swap_add16(h[2 * u], 2 * u + 1 < H ? h[2 * u + 1] : 0.0);
+        s = rotate_add<0x128>(s);   // row_ror 8, 4, 2, 1
+        s = rotate_add<0x124>(s);
+        s = rotate_add<0x122>(s);
+        out[u] = rotate_add<0x121>(s);
+    }
+}
+
 // One thread per stored quartet.  Lists are sorted by bra pair, so a wave
 // usually shares one bra pair: then the bra-side J block is summed across the
 // wave and written with one atomic per element instead of 64 colliding ones.
@@ -353,13 +398,21 @@ __device__ __forceinline__ void jk_tile_item(const JkGroupArgs& g, const JkClass
             uf.digest(a.l32, drows, krows, sbra, d12, j12, tile);
         }
     }
+    {
+        double flat[TA * TB], sum[(TA * TB + 3) / 4];
 #pragma unroll
-    for (int x = 0; x < TA; ++x)
+        for (int t = 0; t < TA * TB; ++t) flat[t] = 4.0 * j12[t / TB][t % TB];
+        wave_sums(flat, sum);
+        if ((tid & 15) == 0) {
+            const int row = (tid >> 4) & 3, first = row == 1 ? 2 : (row == 2 ? 1 : row);
 #pragma unroll
-        for (int y = 0; y < TB; ++y) {
-            const double s = wave_sum(4.0 * j12[x][y]);
-            if ((tid & 63) == 0 && s != 0.0) atomic_addd(&Jm[(size_t)(o1 + a0 + x) * n + o2 + b0 + y], s);
+            for (int u = 0; u < (TA * TB + 3) / 4; ++u) {
+                const int t = 4 * u + first;
+                if (t < TA * TB && sum[u] != 0.0)
+                    atomic_addd(&Jm[(size_t)(o1 + a0 + t / TB) * n + o2 + b0 + t % TB], sum[u]);
+            }
         }
+    }
     __syncthreads();
     double* const ka = Km + (size_t)(o1 + a0) * n;
     double* const kb = Km + (size_t)(o2 + b0) * n;
