@@ -61,17 +61,6 @@ struct EriArgs {
     double scatt_S = 0.0;   // momentum transfer of the scattering operator (OP = 1 kernels)
 };
 
-// Several classes in one launch: blocks [block0[j], block0[j + 1]) run
-// class slot which[j] (eri_fused_k) on quartets cls[j].
-#define ERI_MAXFUSED 8
-template <typename real>
-struct EriFusedArgs {
-    EriArgs<real> cls[ERI_MAXFUSED];
-    int which[ERI_MAXFUSED];
-    int block0[ERI_MAXFUSED + 1];
-    int n;
-};
-
 struct OneeArgs {
     const int* pair_list;
     const PairHdr* pairs;
@@ -214,9 +203,6 @@ __device__ __forceinline__ void boys_eval(float T, float* F)
 #define BOYS_COLS(L) ((L) > 0 ? BOYS_TERMS + 1 : BOYS_TERMS)
 #define BOYS_LDS_DOUBLES(L) (BOYS_NPTS * BOYS_COLS(L))
 
-static __device__ const double boys_inv_fact[BOYS_TERMS] = {
-    1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320};
-
 // The class kernels copy a prepared image of those LDS rows (generated per
 // order L from boys_table.inc): a coalesced copy, two doubles a load.
 __device__ __forceinline__ void boys_stage_copy(double* __restrict__ s, const double* __restrict__ src, const int n)
@@ -225,19 +211,6 @@ __device__ __forceinline__ void boys_stage_copy(double* __restrict__ s, const do
     double2* s2 = (double2*)s;
     for (int e = threadIdx.x; e < n / 2; e += blockDim.x) s2[e] = src2[e];
     if ((n & 1) && threadIdx.x == 0) s[n - 1] = src[n - 1];
-    __syncthreads();
-}
-
-// The same rows formed from boys_table at run time (the fused launch, whose
-// blocks run classes of different orders).
-__device__ __forceinline__ void boys_stage(double* __restrict__ s, const int L)
-{
-    const int W = BOYS_COLS(L);
-#pragma unroll 1
-    for (int e = threadIdx.x; e < BOYS_NPTS * W; e += blockDim.x) {
-        const int k = e / W, c = e - k * W;
-        s[e] = c < BOYS_TERMS ? boys_table[k * BOYS_NCOL + L + c] * boys_inv_fact[c] : exp(-(k * BOYS_STEP));
-    }
     __syncthreads();
 }
 

@@ -297,15 +297,6 @@ size_t eri_scratch_2222_mix();
 void eri_run_2222_s(const EriArgs<double>&, hipStream_t);
 size_t eri_scratch_2222_s();
 void onee_fused_run(const OneeFusedArgs& a, hipStream_t st);
-// classes of the fused heavy-class launch: slot in eri_fused_k, or -1
-#define ERI_NFUSED 0
-static const int eri_fused_slot[ERI_NCLASS] = {
-  -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1, -1
-};
-void eri_fused_run_d(const EriFusedArgs<double>&, hipStream_t);
-void eri_fused_run_f(const EriFusedArgs<float>&, hipStream_t);
-// both precisions' heavy classes in one launch (FP64 blocks first)
-void eri_fused_run_mix(const EriFusedArgs<double>&, const EriFusedArgs<float>&, hipStream_t);
 // la, lb, lc, ld, components, bra pair class, ket pair class
 static const int eri_class_table[ERI_NCLASS][7] = {
   {0, 0, 0, 0, 1, 0, 0},

@@ -438,8 +438,12 @@ def gen_onee(la, lb):
     return "\n".join(lines)
 
 
+_written = set()
+
+
 def _write_if_changed(path, text):
     """Keep mtimes of unchanged generated files so incremental builds skip them."""
+    _written.add(os.path.basename(path))
     if os.path.exists(path):
         with open(path) as fh:
             if fh.read() == text:
@@ -477,12 +481,6 @@ def jk_group(la, lb, lc, ld):
     if (la, lb, lc, ld) in ((2, 2, 2, 2), (2, 0, 1, 1)):
         return 2          # few rows, but the registers of the 3 x 3 tiles
     return next(g for g, (lo, hi) in enumerate(JK_GROUPS) if lo <= ta + tb <= hi)
-
-
-# classes whose kernels spill (scratch) with this generator's code would
-# share one fused launch on the caller's stream (scratch is sized per hardware
-# queue); with the output split above none does
-FUSED = []
 
 
 def boys_rows(here):
@@ -609,48 +607,6 @@ def main():
                "void jk_group_run_%d(const JkGroupArgs& g, int blocks, int block, size_t lds, hipStream_t st)" % g,
                "{ hipLaunchKernelGGL(jk_group_kernel_%d, dim3(blocks), dim3(block), lds, st, g); }" % g]
         _write_if_changed(os.path.join(gdir, "jk_group_%d.hip" % g), "\n".join(js) + "\n")
-    # the heavy classes (their one-thread-per-quartet kernels use scratch)
-    # in one launch: the block index selects the class, so they run side by
-    # side on one queue instead of one after another
-    fz = ["// generated by gen_eri.py -- do not edit", '#include "../eri_common.h"']
-    fz += ['#include "body_%s.h"' % t for t in FUSED]
-    fz.append("template <typename real>")
-    fz.append("__device__ __forceinline__ void eri_fused_block(const EriFusedArgs<real>& a, int b)")
-    fz.append("{")
-    fz.append("  int j = 0;")
-    fz.append("  while (j + 1 < a.n && b >= a.block0[j + 1]) ++j;")
-    fz.append("  const int q = (b - a.block0[j]) * ERI_BLOCK + threadIdx.x;")
-    fz.append("  __shared__ __align__(16) double btab[BOYS_LDS_DOUBLES(1)];   // the widest rows")
-    fz.append("  int L = 0;   // Boys order of the block's class")
-    fz.append("  switch (a.which[j]) {")
-    for k, t in enumerate(FUSED):
-        fz.append("  case %d: L = %d; break;" % (k, sum(int(ch) for ch in t)))
-    fz.append("  default: break;")
-    fz.append("  }")
-    fz.append("  boys_stage(btab, L);")
-    fz.append("  switch (a.which[j]) {")
-    for k, t in enumerate(FUSED):
-        fz.append("  case %d: eri_body_%s<real>(a.cls[j], q, btab); break;" % (k, t))
-    fz.append("  default: break;")
-    fz.append("  }")
-    fz.append("}")
-    fz.append("template <typename real>")
-    fz.append("__global__ void __launch_bounds__(ERI_BLOCK) eri_fused_k(const EriFusedArgs<real> a)")
-    fz.append("{ eri_fused_block<real>(a, blockIdx.x); }")
-    fz.append("__global__ void __launch_bounds__(ERI_BLOCK) eri_fused_mix_k(const EriFusedArgs<double> d, "
-              "const EriFusedArgs<float> f)")
-    fz.append("{")
-    fz.append("  const int nd = d.n > 0 ? d.block0[d.n] : 0;")
-    fz.append("  if ((int)blockIdx.x < nd) eri_fused_block<double>(d, blockIdx.x);")
-    fz.append("  else eri_fused_block<float>(f, blockIdx.x - nd);")
-    fz.append("}")
-    fz.append("void eri_fused_run_mix(const EriFusedArgs<double>& d, const EriFusedArgs<float>& f, hipStream_t st)")
-    fz.append("{ const int nb = (d.n > 0 ? d.block0[d.n] : 0) + (f.n > 0 ? f.block0[f.n] : 0);")
-    fz.append("  if (nb > 0) hipLaunchKernelGGL(eri_fused_mix_k, dim3(nb), dim3(ERI_BLOCK), 0, st, d, f); }")
-    for rn, rt in (("d", "double"), ("f", "float")):
-        fz.append("void eri_fused_run_%s(const EriFusedArgs<%s>& a, hipStream_t st)" % (rn, rt))
-        fz.append("{ if (a.n > 0) hipLaunchKernelGGL(eri_fused_k<%s>, dim3(a.block0[a.n]), dim3(ERI_BLOCK), 0, st, a); }" % rt)
-    _write_if_changed(os.path.join(gdir, "eri_fused.hip"), "\n".join(fz) + "\n")
     onee = ["// generated by gen_eri.py -- do not edit", '#include "../eri_common.h"']
     for la, lb in PAIRS:
         onee.append(gen_onee(la, lb))
@@ -671,6 +627,9 @@ def main():
     onee.append("void onee_fused_run(const OneeFusedArgs& a, hipStream_t st)")
     onee.append("{ if (a.block0[6] > 0) hipLaunchKernelGGL(onee_fused_k, dim3(a.block0[6]), dim3(128), 0, st, a); }")
     _write_if_changed(os.path.join(gdir, "onee.hip"), "\n".join(onee) + "\n")
+    for f in os.listdir(gdir):   # of an older generator
+        if f.endswith((".hip", ".h")) and f not in _written:
+            os.remove(os.path.join(gdir, f))
     # dispatch header
     d = ["// generated by gen_eri.py -- do not edit", "#pragma once", '#include "jk_common.h"',
          "#define ERI_NCLASS %d" % len(CLASSES)]
@@ -687,16 +646,6 @@ def main():
         d.append("void eri_run_%s_s(const EriArgs<double>&, hipStream_t);" % tag)
         d.append("size_t eri_scratch_%s_s();" % tag)
     d.append("void onee_fused_run(const OneeFusedArgs& a, hipStream_t st);")
-    d.append("// classes of the fused heavy-class launch: slot in eri_fused_k, or -1")
-    d.append("#define ERI_NFUSED %d" % len(FUSED))
-    d.append("static const int eri_fused_slot[ERI_NCLASS] = {")
-    d.append("  " + ", ".join(str(FUSED.index("%d%d%d%d" % t[:4])) if "%d%d%d%d" % t[:4] in FUSED else "-1"
-                              for t in table))
-    d.append("};")
-    d.append("void eri_fused_run_d(const EriFusedArgs<double>&, hipStream_t);")
-    d.append("void eri_fused_run_f(const EriFusedArgs<float>&, hipStream_t);")
-    d.append("// both precisions' heavy classes in one launch (FP64 blocks first)")
-    d.append("void eri_fused_run_mix(const EriFusedArgs<double>&, const EriFusedArgs<float>&, hipStream_t);")
     d.append("// la, lb, lc, ld, components, bra pair class, ket pair class")
     d.append("static const int eri_class_table[ERI_NCLASS][7] = {")
     for la, lb, lc, ld, ncomp, X, Y, nbody in table:

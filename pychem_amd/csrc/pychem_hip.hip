@@ -455,7 +455,7 @@ struct pq_basis {
     // caller's stream, four streams fill the process's four hardware queues.
     // J/K: jk_nstreams streams, the caller's one of them (C20H42: 1.24 ms on
     // one, 1.21 on four).  Schwarz and ERI passes: eri_nstreams side
-    // streams beside the caller's, which runs the fused heavy classes.
+    // streams beside the caller's, which runs the classes that use scratch.
     int jk_nstreams = 4;
     int eri_nstreams = 3;
     hipStream_t jk_side[4] = {};
@@ -1012,9 +1012,9 @@ extern "C" int pq_schwarz(pq_basis* b, double* pair_bound_host, void* stream)
         HIPCHK(hipMemcpyAsync(dq.p, hq.data(), sizeof(int2) * nq_all, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(dids.p, hids.data(), sizeof(int) * nq_all, hipMemcpyHostToDevice, st));
     }
-    // the light diagonal classes on the side streams, the heavy ones (their
-    // kernels use scratch) in one fused launch on the caller's stream; each
-    // class's bounds are extracted on the stream that computed it
+    // the diagonal classes on the side streams, those whose kernels use
+    // scratch on the caller's; each class's bounds are extracted on the stream
+    // that computed it
     const int ns = std::min(4, std::max(1, b->eri_nstreams));
     if (ns > 1) {
         if (ensure_jk_streams(b)) return -1;
@@ -1028,42 +1028,19 @@ extern "C" int pq_schwarz(pq_basis* b, double* pair_bound_host, void* stream)
                            (const PairHdr*)b->d_pairs.p, b->any_spher ? (const int*)b->d_spher.p : (const int*)nullptr,
                            (double*)b->d_bound.p);
     };
-    EriFusedArgs<double> fd = {};
-    int nf = 0, side = 0;
-    int hcls[ERI_MAXFUSED], hn[ERI_MAXFUSED];
-    size_t hoq[ERI_MAXFUSED], hov[ERI_MAXFUSED];
-    fd.block0[0] = 0;
+    int side = 0;
     size_t oq = 0, ov = 0;
     for (int X = 0; X < 6; ++X) {
         const int n = (int)b->class_pairs[X].size();
         if (!n) continue;
         const int cls = class_of_pair_classes(X, X);
-        const int ncomp = eri_class_table[cls][4];
-        const int2* q = (const int2*)dq.p + oq;
         double* v = (double*)dv.p + ov;
-        if (eri_fused_slot[cls] >= 0 && nf < ERI_MAXFUSED) {
-            fd.cls[nf] = EriArgs<double>{q, (const PairHdr*)b->d_pairs.p, (const PrimPair<double>*)b->d_prims.p, v, n};
-            fd.which[nf] = eri_fused_slot[cls];
-            fd.block0[nf + 1] = fd.block0[nf] + (n + ERI_BLOCK - 1) / ERI_BLOCK;
-            hcls[nf] = cls;
-            hn[nf] = n;
-            hoq[nf] = oq;
-            hov[nf] = ov;
-            ++nf;
-        } else {
-            hipStream_t sk = (ns > 1 && class_scratch(b, cls, false) == 0) ? b->jk_side[side++ % ns] : st;
-            if (run_class<double>(b, cls, q, n, v, sk)) return -1;
-            extract(cls, n, oq, ov, sk);
-        }
+        hipStream_t sk = (ns > 1 && class_scratch(b, cls, false) == 0) ? b->jk_side[side++ % ns] : st;
+        if (run_class<double>(b, cls, (const int2*)dq.p + oq, n, v, sk)) return -1;
+        extract(cls, n, oq, ov, sk);
         HIPCHK(hipGetLastError());
         oq += n;
-        ov += (size_t)n * ncomp;
-    }
-    if (nf) {
-        fd.n = nf;
-        eri_fused_run_d(fd, st);
-        for (int j = 0; j < nf; ++j) extract(hcls[j], hn[j], hoq[j], hov[j], st);
-        HIPCHK(hipGetLastError());
+        ov += (size_t)n * eri_class_table[cls][4];
     }
     if (ns > 1)
         for (int k = 0; k < ns; ++k) {
@@ -1559,8 +1536,7 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
 // primitive quartets x components) and join back, so that the classes
 // overlap.  Kernels that spill (per-lane scratch: the runtime sizes scratch
 // per hardware queue for a full device of waves) stay on `st`, the one queue
-// that always carried them; the heavy classes whose kernels spill run there
-// as one fused launch, both precisions together.
+// that always carried them.
 extern "C" int pq_eri_compute(pq_basis* b, void* stream)
 {
     if (!b) return fail("pq_eri_compute: null basis");
@@ -1605,40 +1581,9 @@ extern "C" int pq_eri_compute(pq_basis* b, void* stream)
             }
         return 0;
     };
-    // the heavy classes (their kernels use scratch): one launch on the
-    // caller's stream, both precisions, the block index selects the class
-    {
-        EriFusedArgs<double> fd = {};
-        EriFusedArgs<float> ff = {};
-        for (int c = 0; c < ERI_NCLASS; ++c) {
-            if (eri_fused_slot[c] < 0) continue;
-            if (b->store64[c].nq) {
-                fd.cls[fd.n] = args_d(c);
-                fd.which[fd.n] = eri_fused_slot[c];
-                fd.block0[fd.n + 1] = fd.block0[fd.n] + (b->store64[c].nq + ERI_BLOCK - 1) / ERI_BLOCK;
-                ++fd.n;
-            }
-            if (b->store32[c].nq) {
-                ff.cls[ff.n] = args_f(c);
-                ff.which[ff.n] = eri_fused_slot[c];
-                ff.block0[ff.n + 1] = ff.block0[ff.n] + (b->store32[c].nq + ERI_BLOCK - 1) / ERI_BLOCK;
-                ++ff.n;
-            }
-        }
-        if (fd.n || ff.n) {
-            for (int c = 0; c < ERI_NCLASS; ++c)
-                if (eri_fused_slot[c] >= 0 && mark(c, 0, st)) return -1;
-            if (ff.n) eri_fused_run_mix(fd, ff, st);
-            else eri_fused_run_d(fd, st);
-            HIPCHK(hipGetLastError());
-            for (int c = 0; c < ERI_NCLASS; ++c)
-                if (eri_fused_slot[c] >= 0 && mark(c, 1, st)) return -1;
-        }
-    }
     double load[4] = {0.0, 0.0, 0.0, 0.0};
     for (const auto& o : order) {
         const int c = o.second;
-        if (eri_fused_slot[c] >= 0) continue;
         int k = 0;
         for (int t = 1; t < ns; ++t)
             if (load[t] < load[k]) k = t;
