@@ -188,20 +188,30 @@ __device__ __forceinline__ void boys_eval(float T, float* F)
     }
 }
 
-// The class kernels read the Taylor coefficients from LDS: a lookup gathers
-// 9 doubles at a lane-dependent row, and from global memory that costs three
-// scattered 16-byte loads per lane and primitive quartet (the (ss|ss) and
-// (ps|ss) kernels were bound by them).  boys_stage copies, for every grid
-// point T_k, the Taylor coefficients F_{L+c}(T_k) / c!, c = 0..8 (the only
-// ones F_L's expansion reads, in both precisions), and for L > 0 also
-// e^{-T_k}, into the block's LDS: BOYS_COLS(L) doubles per point.  With the
-// divided coefficients the expansion is a plain Horner chain of fused
-// multiply-adds, and e^{-T} = e^{-T_k} e^{T_k - T} costs a degree-8 Taylor
-// polynomial of e^x on |x| <= 0.05 (remainder below 6e-18 relative) instead
-// of a full exponential.
+// The class kernels read the polynomial coefficients from LDS: a lookup
+// gathers 8 or 9 doubles at a lane-dependent row, and from global memory that
+// costs scattered 16-byte loads per lane and primitive quartet (the (ss|ss)
+// and (ps|ss) kernels were bound by them).  The image (boys_stage_copy) holds
+// BOYS_COLS doubles per grid point T_k, coefficients of x^c, x = T_k - T,
+// divided by c!, so that the expansion is a Horner chain of fused
+// multiply-adds:
+//   L = 0                    F_0, degree 7
+//   L <= BOYS_PAIR_MAX       F_{L-1}, degree 8; its derivative in x is F_L
+//   above                    F_L, degree 8, and e^{-T_k}
+// The first two are Taylor polynomials of one degree more less their top
+// Chebyshev component: off by 4e-19, below the 5e-18 of the degree 8 Taylor
+// polynomial they replace.  Rows are an odd number (5) of 16-byte units: a
+// random row then spreads over all banks and is read 16 bytes at a time, 46
+// cycles of the CU's LDS for the 8 doubles of a wave, where 9 doubles in rows
+// of 9 took 96 with 8-byte reads; (ss|ss), whose four SIMDs can issue a
+// primitive quartet in some 170 cycles, was bound by those 4 x 96.  The pair
+// of orders from one polynomial and the shorter far branch leave (ps|ss) 79
+// vector instructions of 124 where a wave takes both branches.  The pass over
+// C20H42's lists went from 3.13 to 2.87 ms, over C14H30's from 1.72 to 1.58.
 #define BOYS_TERMS 9
-#define BOYS_COLS(L) ((L) > 0 ? BOYS_TERMS + 1 : BOYS_TERMS)
-#define BOYS_LDS_DOUBLES(L) (BOYS_NPTS * BOYS_COLS(L))
+#define BOYS_COLS 10
+#define BOYS_LDS_DOUBLES (BOYS_NPTS * BOYS_COLS)
+#define BOYS_PAIR_MAX 5
 
 // The class kernels copy a prepared image of those LDS rows (generated per
 // order L from boys_table.inc): a coalesced copy, two doubles a load.
@@ -214,52 +224,80 @@ __device__ __forceinline__ void boys_stage_copy(double* __restrict__ s, const do
     __syncthreads();
 }
 
-// 1/sqrt(s) for positive normal s: the hardware estimate and two Newton
-// steps y <- y + y (1 - s y^2) / 2, each of which squares the relative error.
+// 1/sqrt(s) for positive normal s: the hardware estimate y (2^-22 relative
+// or better) and the next two terms of its error series,
+// y (1 - e)^{-1/2} = y + y e (1/2 + 3/8 e) + O(e^3), e = 1 - s y^2.
 __device__ __forceinline__ double rsqrt_nr(const double s)
 {
-    double y = __builtin_amdgcn_rsq(s);
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const double e = fma(-s * y, 0.5 * y, 0.5);
-        y = fma(y, e, y);
-    }
-    return y;
+    const double y = __builtin_amdgcn_rsq(s);
+    const double e = fma(-s * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// e^{-T} for T >= BOYS_TMAX, to about 2e-10 relative: n = rint(T / ln 2),
-// r = T - n ln 2 in [-0.35, 0.35], e^{-r} by its degree-8 Taylor polynomial,
-// scaled by 2^-n.  In the upward recursion above T = 36 the e^{-T} term is
-// at most 8e-9 of (2m+1) F_m for m <= 7, so this accuracy leaves F_m exact to
-// rounding.  2^-n underflows to 0 where e^{-T} does.
+// e^{-T} for T >= BOYS_TMAX: n = rint(T / ln 2), r = T - n ln 2 in [-0.35,
+// 0.35], e^{-r} by its Taylor polynomial of degree DEG, scaled by 2^-n.  In
+// the upward recursion above T = 36 the e^{-T} term is at most 1.6e-15,
+// 3.7e-14, 5e-13, 5.6e-12, 4.4e-11 and, for m = 7, 8e-9 of (2m+1) F_m, m = 0,
+// 1, ..., 4; a polynomial good to 6e-4 (degree 3), 4e-5, 2.4e-6, 1.2e-7, 5e-9
+// and 2e-10 (degree 8) leaves F_{m+1} exact to rounding.  2^-n underflows to
+// 0 where e^{-T} does.
+template <int DEG>
 __device__ __forceinline__ double exp_neg_tail(const double T)
 {
-    const double n = rint(T * 1.4426950408889634);
-    const double r = fma(-n, 0.69314718055994531, T);
+    const double n = rint(T * -1.4426950408889634);
+    const double r = fma(n, 0.69314718055994531, T);
     constexpr double c[9] = {1.0, -1.0, 1.0 / 2, -1.0 / 6, 1.0 / 24, -1.0 / 120, 1.0 / 720, -1.0 / 5040, 1.0 / 40320};
-    double p = c[8];
+    double p = c[DEG];
 #pragma unroll
-    for (int j = 7; j >= 0; --j) p = fma(p, r, c[j]);
-    return ldexp(p, -(int)fmin(n, 2000.0));
+    for (int j = DEG - 1; j >= 0; --j) p = fma(p, r, c[j]);
+    return ldexp(p, (int)fmax(n, -2000.0));
 }
 
 template <int L>
 __device__ __forceinline__ void boys_eval_s(double T, double* F, const double* __restrict__ s)
 {
     if (T < BOYS_TMAX) {
-        const int k = __double2int_rn(T * BOYS_INV_STEP);
-        const double x = k * BOYS_STEP - T;
-        const double* row = s + k * BOYS_COLS(L);
-        double f = row[8];
+        // 1.5 x 2^52 rounds to the nearest grid point, k in the low word
+        const double t = fma(T, BOYS_INV_STEP, 6755399441055744.0);
+        const double x = fma(t - 6755399441055744.0, BOYS_STEP, -T);
+        const double2* row = (const double2*)s + __umul24(__double2loint(t), BOYS_COLS / 2);
+        double c[BOYS_COLS];
 #pragma unroll
-        for (int j = 7; j >= 0; --j) f = fma(f, x, row[j]);
-        F[L] = f;
-        if (L > 0) {
-            constexpr double c[8] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040};
+        for (int j = 0; j < (L == 0 ? 4 : 5); ++j) {
+            const double2 v = row[j];
+            c[2 * j] = v.x;
+            c[2 * j + 1] = v.y;
+        }
+        if constexpr (L == 0) {
+            double f = c[7];
+#pragma unroll
+            for (int j = 6; j >= 0; --j) f = fma(f, x, c[j]);
+            F[0] = f;
+        } else if constexpr (L <= BOYS_PAIR_MAX) {
+            double d = c[8], f = fma(c[8], x, c[7]);
+#pragma unroll
+            for (int j = 6; j >= 0; --j) {
+                d = fma(d, x, f);
+                f = fma(f, x, c[j]);
+            }
+            F[L] = d;
+            F[L - 1] = f;
+            if constexpr (L > 1) {   // e^{-T} = (2m+1) F_m - 2T F_{m+1}
+                const double t2 = 2.0 * T;
+                const double e = fma(-t2, d, (2 * L - 1) * f);
+#pragma unroll
+                for (int m = L - 2; m >= 0; --m) F[m] = fma(t2, F[m + 1], e) * (1.0 / (2 * m + 1));
+            }
+        } else {
+            double f = c[8];
+#pragma unroll
+            for (int j = 7; j >= 0; --j) f = fma(f, x, c[j]);
+            F[L] = f;
+            constexpr double w[8] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040};
             double ex = 1.0 / 40320;
 #pragma unroll
-            for (int j = 7; j >= 0; --j) ex = fma(ex, x, c[j]);
-            const double e = row[BOYS_TERMS] * ex;
+            for (int j = 7; j >= 0; --j) ex = fma(ex, x, w[j]);
+            const double e = c[BOYS_TERMS] * ex;
             const double t2 = 2.0 * T;
 #pragma unroll
             for (int m = L - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0 / (2 * m + 1));
@@ -268,7 +306,7 @@ __device__ __forceinline__ void boys_eval_s(double T, double* F, const double* _
         const double y = rsqrt_nr(T);
         F[0] = 0.88622692545275801365 * y;
         if (L > 0) {
-            const double e = exp_neg_tail(T);
+            const double e = exp_neg_tail<(L <= 5 ? L + 2 : 8)>(T);
             const double h = 0.5 * y * y;
 #pragma unroll
             for (int m = 0; m < L; ++m) F[m + 1] = ((2 * m + 1) * F[m] - e) * h;
@@ -282,16 +320,36 @@ __device__ __forceinline__ void boys_eval_s(float T, float* F, const double* __r
     if (T < (float)BOYS_TMAX) {
         const int k = __float2int_rn(T * (float)BOYS_INV_STEP);
         const float x = k * (float)BOYS_STEP - T;
-        const double* row = s + k * BOYS_COLS(L);
-        float f = (float)row[5];
+        const double2* row = (const double2*)s + __umul24(k, BOYS_COLS / 2);
+        float c[8];
 #pragma unroll
-        for (int j = 4; j >= 0; --j) f = fmaf(f, x, (float)row[j]);
-        F[L] = f;
-        if (L > 0) {
+        for (int j = 0; j < (L == 0 || L > BOYS_PAIR_MAX ? 3 : 4); ++j) {
+            const double2 v = row[j];
+            c[2 * j] = (float)v.x;
+            c[2 * j + 1] = (float)v.y;
+        }
+        constexpr int M = L == 0 || L > BOYS_PAIR_MAX ? L : L - 1;   // the order whose polynomial the row holds
+        float f, d = 0.0f;
+        if constexpr (M < L) {
+            d = c[6];
+            f = fmaf(c[6], x, c[5]);
+#pragma unroll
+            for (int j = 4; j >= 0; --j) {
+                d = fmaf(d, x, f);
+                f = fmaf(f, x, c[j]);
+            }
+            F[L] = d;
+        } else {
+            f = c[5];
+#pragma unroll
+            for (int j = 4; j >= 0; --j) f = fmaf(f, x, c[j]);
+        }
+        F[M] = f;
+        if (M > 0) {
             const float e = __expf(-T);
             const float t2 = 2.0f * T;
 #pragma unroll
-            for (int m = L - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0f / (2 * m + 1));
+            for (int m = M - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0f / (2 * m + 1));
         }
     } else {
         boys_eval<L>(T, F);

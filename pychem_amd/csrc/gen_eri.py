@@ -24,6 +24,8 @@ Run: python pychem_amd/csrc/gen_eri.py   (writes eri_classes.inc next to it)
 """
 import math
 import os
+import re
+from fractions import Fraction
 
 PAIRS = [(0, 0), (1, 0), (1, 1), (2, 0), (2, 1), (2, 2)]   # pair classes (primary, secondary)
 CLASSES = [(X, Y) for X in range(len(PAIRS)) for Y in range(X + 1)]
@@ -83,6 +85,7 @@ def gen_eri_class(la, lb, lc, ld, asel=None, csel=None, suffix=""):
     em = Emitter()
 
     flops = {"vrr": 0, "contract": 0, "hrr": 0}
+    terms = {}           # summands of each recurrence
 
     def vrr(e, f, m):
         # flops priced as the reference's two_electron_vrr.c:92-109: 6 for the
@@ -118,6 +121,8 @@ def gen_eri_class(la, lb, lc, ld, asel=None, csel=None, suffix=""):
             expr = " + ".join(t)
         em.emit("const real %s = %s;" % (name, expr))
         em.done.add(key)
+        if not (lev(e) == 0 and lev(f) == 0):
+            terms[name] = t
         return name
 
     def reach(a, b):     # the [e0| components the bra HRR of (a b| reads
@@ -133,13 +138,24 @@ def gen_eri_class(la, lb, lc, ld, asel=None, csel=None, suffix=""):
     for e in ecomps:
         for f in fcomps:
             acc_names[(e, f)] = "c%s_%s" % (nm(e), nm(f))
-    # primitive-quartet body
+    # primitive-quartet body; a target no other recurrence reads is added to
+    # its accumulator term by term, each a fused multiply-add
+    targets = {}
     for e in ecomps:
         for f in fcomps:
-            v = vrr(e, f, 0)
-            em.emit("%s += %s;" % (acc_names[(e, f)], v))
+            targets[vrr(e, f, 0)] = acc_names[(e, f)]
             flops["contract"] += 3   # two_electron_contract.c:45
-    body = em.lines
+    read = {w for l in em.lines for w in re.findall(r"v\w+", l.split(" = ")[1])}
+    body = []
+    for line in em.lines:
+        v = line.split(" = ")[0].split()[-1]
+        if v in targets and v in terms and v not in read:
+            body += ["%s%s += %s;" % (em.ind, targets[v], t) for t in terms[v]]
+        else:
+            body.append(line)
+            if v in targets:
+                body.append("%s%s += %s;" % (em.ind, targets[v], v))
+    nbody = len(em.lines) + len(targets)
 
     # HRR (post loop)
     hr = Emitter(indent="  ")
@@ -221,7 +237,7 @@ def gen_eri_class(la, lb, lc, ld, asel=None, csel=None, suffix=""):
         out += ["    }", "  }"]
         return out
 
-    if len(body) <= UNIFORM_MAX_BODY:
+    if nbody <= UNIFORM_MAX_BODY:
         lines.append("  if (__all(pr.x == __builtin_amdgcn_readfirstlane(pr.x))) {")
         lines.append("    const int bn = __builtin_amdgcn_readfirstlane(bh.n);")
         lines.append("    const ERI_CONST PrimPair<double>* __restrict__ bp =")
@@ -239,7 +255,7 @@ def gen_eri_class(la, lb, lc, ld, asel=None, csel=None, suffix=""):
     lines.append("}")
     gen_eri_class.flops = dict(flops, boys=L + 1)
     gen_eri_class.naccum = len(acc_names)
-    return "\n".join(lines), ncomp, len(body)
+    return "\n".join(lines), ncomp, nbody
 
 
 # Classes whose one-thread-per-quartet kernel would hold too many [e0|f0]
@@ -494,18 +510,43 @@ def boys_rows(here):
     return step, [vals[i:i + ncol] for i in range(0, len(vals), ncol)]
 
 
+# Up to this Boys order a class takes F_L and F_{L-1} from one polynomial
+# (boys_eval_s); must equal BOYS_PAIR_MAX of eri_common.h.
+BOYS_PAIR_MAX = 5
+
+
+def economised(c, h):
+    """The polynomial sum_j c[j] x^j less its top Chebyshev component on
+    |x| <= h: one degree lower, off by c[n] h^n / 2^(n-1) at most."""
+    n = len(c) - 1
+    t0, t1 = [1], [0, 1]                        # Chebyshev T_0, T_1, ..., T_n
+    for _ in range(n - 1):
+        t2 = [0] + [2 * v for v in t1]
+        for k, v in enumerate(t0):
+            t2[k] -= v
+        t0, t1 = t1, t2
+    return [c[k] - c[n] * h ** (n - k) * t1[k] / 2 ** (n - 1) for k in range(n)]
+
+
 def boys_lds_table(L, step, rows):
-    """The LDS image a class kernel of Boys order L stages (boys_stage_copy):
-    per grid point the Taylor coefficients F_{L+c}(T_k) / c!, c = 0..8, and
-    for L > 0 e^{-T_k} (T_k the double k * step, as the kernel forms it)."""
+    """The LDS image a class kernel of Boys order L stages (boys_stage_copy),
+    10 doubles per grid point T_k: polynomial coefficients of F_0(T_k - x)
+    (L = 0: 8) or F_{L-1}(T_k - x) (to BOYS_PAIR_MAX: 9), the Taylor series
+    economised by one degree; above that the 9 Taylor coefficients
+    F_{L+c}(T_k) / c! and e^{-T_k} (T_k the double k * step, as the kernel
+    forms it)."""
     out = []
+    h = Fraction(step) / 2
     for k, r in enumerate(rows):
-        out += [r[L + c] * (1.0 / math.factorial(c)) for c in range(9)]
-        if L > 0:
-            out.append(math.exp(-(k * step)))
+        if L <= BOYS_PAIR_MAX:
+            n, m = (8, 0) if L == 0 else (9, L - 1)
+            c = economised([Fraction(r[m + j]) / math.factorial(j) for j in range(n + 1)], h)
+            out += [float(v) for v in c] + [0.0] * (10 - n)
+        else:
+            out += [r[L + c] * (1.0 / math.factorial(c)) for c in range(9)] + [math.exp(-(k * step))]
     name = "boys_lds_L%d" % L
     lines = ["// Boys coefficients staged in LDS by the class kernels of order %d" % L,
-             "static __device__ __align__(16) const double %s[BOYS_LDS_DOUBLES(%d)] = {" % (name, L)]
+             "static __device__ __align__(16) const double %s[BOYS_LDS_DOUBLES] = {" % name]
     for i in range(0, len(out), 6):
         lines.append("  " + ", ".join("%.17e" % v for v in out[i:i + 6]) + ",")
     lines.append("};")
@@ -541,8 +582,8 @@ def main():
                "template <typename real>",
                "__global__ void __launch_bounds__(ERI_BLOCK, ERI_MINW) eri_k%s(const EriArgs<real> args)" % tag,
                "{",
-               "  __shared__ __align__(16) double btab[BOYS_LDS_DOUBLES(%d)];" % Lc,
-               "  boys_stage_copy(btab, %s, BOYS_LDS_DOUBLES(%d));" % (btname, Lc),
+               "  __shared__ __align__(16) double btab[BOYS_LDS_DOUBLES];",
+               "  boys_stage_copy(btab, %s, BOYS_LDS_DOUBLES);" % btname,
                "  eri_body_%s<real>(args, blockIdx.x * blockDim.x + threadIdx.x, btab);" % tag,
                "}"]
         # both lists of the class in one launch (FP64 blocks first): the FP32
@@ -550,8 +591,8 @@ def main():
         src.append("__global__ void __launch_bounds__(ERI_BLOCK, ERI_MINW) eri_kmix%s(const EriArgs<double> d, "
                    "const EriArgs<float> f, int nb64)" % tag)
         src.append("{")
-        src.append("  __shared__ __align__(16) double btab[BOYS_LDS_DOUBLES(%d)];" % Lc)
-        src.append("  boys_stage_copy(btab, %s, BOYS_LDS_DOUBLES(%d));" % (btname, Lc))
+        src.append("  __shared__ __align__(16) double btab[BOYS_LDS_DOUBLES];")
+        src.append("  boys_stage_copy(btab, %s, BOYS_LDS_DOUBLES);" % btname)
         src.append("  if ((int)blockIdx.x < nb64) eri_body_%s<double>(d, blockIdx.x * blockDim.x + threadIdx.x, btab);" % tag)
         src.append("  else eri_body_%s<float>(f, (blockIdx.x - nb64) * blockDim.x + threadIdx.x, btab);" % tag)
         src.append("}")
