@@ -321,6 +321,10 @@ static const int eri_class_table[ERI_NCLASS][7] = {
   {2, 2, 2, 1, 648, 5, 4},
   {2, 2, 2, 2, 1296, 5, 5},
 };
+// VRR and contraction lines per primitive quartet (of one output group)
+static const int eri_body_lines[ERI_NCLASS] = {
+  2, 8, 27, 24, 79, 227, 21, 70, 200, 152, 51, 170, 252, 366, 305, 101, 340, 353, 172, 411, 955
+};
 // the electron-scattering operator's class kernels (FP64)
 static void (*const eri_table_s[ERI_NCLASS])(const EriArgs<double>&, hipStream_t) = {
   eri_run_0000_s, eri_run_1000_s, eri_run_1010_s, eri_run_1100_s, eri_run_1110_s, eri_run_1111_s, eri_run_2000_s, eri_run_2010_s, eri_run_2011_s, eri_run_2020_s, eri_run_2100_s, eri_run_2110_s, eri_run_2111_s, eri_run_2120_s, eri_run_2121_s, eri_run_2200_s, eri_run_2210_s, eri_run_2211_s, eri_run_2220_s, eri_run_2221_s, eri_run_2222_s

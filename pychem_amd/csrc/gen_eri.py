@@ -692,6 +692,10 @@ def main():
     for la, lb, lc, ld, ncomp, X, Y, nbody in table:
         d.append("  {%d, %d, %d, %d, %d, %d, %d}," % (la, lb, lc, ld, ncomp, X, Y))
     d.append("};")
+    d.append("// VRR and contraction lines per primitive quartet (of one output group)")
+    d.append("static const int eri_body_lines[ERI_NCLASS] = {")
+    d.append("  " + ", ".join(str(t[7]) for t in table))
+    d.append("};")
     d.append("// the electron-scattering operator's class kernels (FP64)")
     d.append("static void (*const eri_table_s[ERI_NCLASS])(const EriArgs<double>&, hipStream_t) = {")
     d.append("  " + ", ".join("eri_run_%d%d%d%d_s" % (t[0], t[1], t[2], t[3]) for t in table))

@@ -397,6 +397,7 @@ struct pq_basis {
     std::vector<long long> mol_pair_off;
     std::vector<int> mol_shell0, mol_nshell;
     std::vector<std::vector<int>> class_pairs;   // pair ids per pair class
+    int class_nmax[6] = {};                      // most primitive pairs of a pair of the class
     std::vector<double> bound;              // per pair Schwarz bound
     int have_bound = 0;
     // two-electron operator of the class kernels: 0 Coulomb, 1 electron
@@ -789,6 +790,7 @@ extern "C" int pq_basis_create_batch(int nmol, int nshell, const int* l, const i
         b->pair_local[(size_t)(b->mol_pair_off[m] + (long long)(sa - s0) * ns + (sb - s0))] = t;
         b->pair_local[(size_t)(b->mol_pair_off[m] + (long long)(sb - s0) * ns + (sa - s0))] = t;
         b->class_pairs[b->pairs[t].pcls].push_back(t);
+        b->class_nmax[b->pairs[t].pcls] = std::max(b->class_nmax[b->pairs[t].pcls], b->pairs[t].n);
     }
     b->npair = (int)b->pairs.size();
     b->nprimpair = (int)nprims;
@@ -1532,23 +1534,33 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
 // All class kernels over the planned lists (the ERI-generation pass).
 // Each class is one launch: its FP64 and FP32 lists (a mixed-precision plan)
 // together, the FP64 blocks first.  The launches fork from `st` onto the
-// side streams (costliest first, each to the least-loaded stream; cost ~
-// primitive quartets x components) and join back, so that the classes
-// overlap.  Kernels that spill (per-lane scratch: the runtime sizes scratch
-// per hardware queue for a full device of waves) stay on `st`, the one queue
-// that always carried them.
+// side streams (the longest expected launch first, each to the least-loaded
+// stream) and join back, so that the classes overlap.  Kernels that spill
+// (per-lane scratch: the runtime sizes scratch per hardware queue for a full
+// device of waves) stay on `st`, the one queue that always carried them.
 extern "C" int pq_eri_compute(pq_basis* b, void* stream)
 {
     if (!b) return fail("pq_eri_compute: null basis");
     hipStream_t st = (hipStream_t)stream;
     if (b->timing && ensure_events(b)) return -1;
+    // A launch lasts about as long as its deepest quartet's chain of dependent
+    // instructions, some 8 cycles each (a lane runs all of a quartet's
+    // primitives: 1296 of (ss|ss) or 81 of (pp|pp) in 6-31G* are 0.4 and
+    // 0.17 ms, however few such quartets there are), plus its share of the
+    // chip, 4 cycles per wave instruction and SIMD.  By work alone the deep
+    // classes with little of it came last and the pass ended in their chains:
+    // C14H30 1.72 ms, in this order 1.58.
     std::vector<std::pair<double, int>> order;
     for (int c = 0; c < ERI_NCLASS; ++c) {
+        const double body = 1.5 * eri_body_lines[c] + 50.0;
+        const int deepest = b->class_nmax[eri_class_table[c][5]] * b->class_nmax[eri_class_table[c][6]];
         double cost = 0.0;
         for (int w = 0; w < 2; ++w) {
             EriClassStore& s = w ? b->store32[c] : b->store64[c];
             b->ev_cls_used[2 * c + w] = 0;
-            if (s.nq) cost += (double)s.nprimq * s.ncomp + (double)s.nq * s.ncomp;
+            if (s.nq)
+                cost += 8.0 * (body * deepest + 20.0 * s.ncomp) +
+                        4.0 / (64 * 1024) * (body * s.nprimq + (200.0 + 8.0 * s.ncomp) * s.nq);
         }
         if (cost > 0.0) order.push_back({cost, c});
     }
