@@ -21,6 +21,7 @@ struct ListArgs {
     const int* bra_seg;          // [nmol + 1] molecule segment starts in bra
     const int* ket_seg;          // [nmol + 1] molecule segment starts in ket
     const long long* ket_npcum;  // [nket + 1] cumulative primitive-pair counts along ket
+    const unsigned* ket_rec;     // [nk] the digestion kernels' ket record (function offsets, same-shell bit)
     const double* bound;         // Schwarz bound per pair id
     const double* bra_bound;     // bound of bra[i], in bra order
     const PairHdr* pairs;
@@ -69,6 +70,7 @@ struct ListJob {
     int nb_items;          // bras whose items are counted (0: class without quartets)
     int has32;             // the class has an FP32 list
     int* ord[2];           // quartet order of the ERI kernels (list_order_batch; NULL: none)
+    unsigned char* bk[2];  // each quartet's bucket in that order (list_fill_batch; NULL: none)
 };
 struct ListBlocks {
     int block0[LIST_MAXJOB + 1];
@@ -84,20 +86,21 @@ struct ScanJob {
 void list_count_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st);
 // one single-workgroup exclusive scan per ScanJob (jobs in device memory)
 void list_scan_batch(const ScanJob* jobs, int n, hipStream_t st);
-// every quartet of every list: jobs' list w = 0, 1 as blocks 2j + w
-void list_fill_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st);
-// per bra of every job (block0 over nb_items): work items of its kets
-void list_items_count_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st);
-// Order in which the ERI kernels visit each list (jobs' q[w], ord[w]; the
-// blocks of list_fill_batch): quartets by descending primitive work
-// (primitive pairs of bra x ket, in half-octave buckets), so that the lanes
-// of a wave loop over about as many primitive quartets as one another.  A
-// counting sort: per-bucket counts, their scan, then each quartet's slot.
-// cnt and cur: ORD_NB ints per list (2 per job); cnt zeroed here.  blk:
-// ceil(nq / (256 ORD_PT)) blocks per list, none for lists without an order.
+// every quartet of every list, jobs' list w = 0, 1 as blocks 2j + w, each of
+// ceil(nq / (256 ORD_PT)) blocks, with the buckets of list_order_batch and
+// cnt, their counts (ORD_NB ints per list, zeroed here)
 #define ORD_NB 32
 #define ORD_PT 16
-void list_order_batch(const ListJob* jobs, const ListBlocks& blk, int* cnt, int* cur, hipStream_t st);
+void list_fill_batch(const ListJob* jobs, const ListBlocks& blk, int* cnt, hipStream_t st);
+// per bra of every job (block0 over nb_items): work items of its kets
+void list_items_count_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st);
+// Order in which the ERI kernels visit each list (jobs' bk[w] -> ord[w]; the
+// blocks and counts of list_fill_batch): quartets by descending primitive work
+// (primitive pairs of bra x ket, in half-octave buckets), so that the lanes
+// of a wave loop over about as many primitive quartets as one another.  A
+// counting sort, in list order within a bucket and block.  cur: ORD_NB ints
+// per list.
+void list_order_batch(const ListJob* jobs, const ListBlocks& blk, const int* cnt, int* cur, hipStream_t st);
 // every work item of every job (block0 over nitems)
 void list_items_fill_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st);
 

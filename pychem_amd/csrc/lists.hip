@@ -119,9 +119,7 @@ __device__ __forceinline__ void list_fill_one(const ListArgs& a, const ListBras&
     const int j = b.j0[i] + (int)(q - b.qs[i]);
     const int P = a.bra[i], Q = a.ket[j];
     quartets[q] = make_int2(P, Q);
-    const PairHdr kh = a.pairs[Q];
-    kets[q] = (unsigned)a.cart_off[kh.s1] | ((unsigned)a.cart_off[kh.s2] << 15) |
-              ((kh.s1 == kh.s2) ? (1u << 30) : 0u) | ((P == Q) ? (1u << 31) : 0u);
+    kets[q] = a.ket_rec[j] | (P == Q ? 1u << 31 : 0u);
 }
 
 __global__ void list_fill_kernel(const ListArgs a, const ListBras b, long long nq, int2* quartets, unsigned* kets)
@@ -178,20 +176,11 @@ __global__ void __launch_bounds__(256) list_count_batch_kernel(const ListJob* jo
     if (i < J.a.nb) list_count_one(J.a, J.b64, J.b32, i);
 }
 
-__global__ void __launch_bounds__(256) list_fill_batch_kernel(const ListJob* jobs, const ListBlocks blk)
+// Bucket of a quartet of `work` primitive quartets: 0 holds the most, half an
+// octave per bucket.
+__device__ __forceinline__ int order_bucket(int work)
 {
-    int q;
-    const int jw = list_job_of(blk, q), j = jw >> 1, w = jw & 1;
-    const ListJob& J = jobs[j];
-    if (q < J.nq[w]) list_fill_one(J.a, w ? J.b32 : J.b64, q, J.q[w], J.k[w]);
-}
-
-// Bucket of quartet i of a list: 0 holds the most primitive quartets (bra
-// pairs x ket pairs), half an octave per bucket.
-__device__ __forceinline__ int order_bucket(const ListJob& J, int w, long long i)
-{
-    const int2 pr = J.q[w][i];
-    const int work = max(1, J.a.pairs[pr.x].n * J.a.pairs[pr.y].n);
+    work = max(1, work);
     const int lg = 31 - __clz(work);                                  // floor(log2 work)
     const int k = 2 * lg + (lg > 0 ? (work >> (lg - 1)) & 1 : 0);   // half-octaves
     return ORD_NB - 1 - min(k, ORD_NB - 1);
@@ -208,22 +197,66 @@ __device__ __forceinline__ int order_job_of(const ListBlocks& blk, int& lb)
     return j;
 }
 
-__global__ void __launch_bounds__(256) list_order_count_kernel(const ListJob* jobs, const ListBlocks blk, int* cnt)
+// lanes of the wave that hold a quartet (ok) of the same bucket as this one
+__device__ __forceinline__ unsigned long long bucket_peers(int bucket, bool ok)
 {
-    __shared__ int h[ORD_NB];
+    unsigned long long m = __ballot(ok);
+#pragma unroll
+    for (int k = 0; (1 << k) < ORD_NB; ++k) {
+        const bool bit = (bucket >> k) & 1;
+        const unsigned long long v = __ballot(bit);
+        m &= bit ? v : ~v;
+    }
+    return m;
+}
+
+// Quartets q0 ... of one list, ORD_PT * 256 to a block: the bras of the
+// block's first and last quartet are searched once, each quartet's bra
+// between them, and what a quartet needs of its ket lies in ket order (one
+// search over all bras and three gathers, each behind the last, per quartet:
+X  Bucket and bucket counts are taken here, where both pairs'
+// primitive counts are at hand.
+__global__ void __launch_bounds__(256) list_fill_batch_kernel(const ListJob* jobs, const ListBlocks blk, int* cnt)
+{
+    __shared__ int h[ORD_NB], ends[2];
     int lb;
     const int jw = order_job_of(blk, lb), w = jw & 1;
     const ListJob& J = jobs[jw >> 1];
+    // copies: the stores below could alias the job
+    const ListArgs a = J.a;
+    const ListBras b = w ? J.b32 : J.b64;
+    const long long q0 = (long long)lb * 256 * ORD_PT, left = J.nq[w] - q0;
+    const int nq = left < 256 * ORD_PT ? (int)left : 256 * ORD_PT;
+    int2* const quartets = J.q[w];
+    unsigned* const kets = J.k[w];
+    unsigned char* const bk = J.bk[w];
     if (threadIdx.x < ORD_NB) h[threadIdx.x] = 0;
+    if (threadIdx.x < 2) ends[threadIdx.x] = last_le(b.qs, a.nb, threadIdx.x ? q0 + nq - 1 : q0);
     __syncthreads();
-    const long long q0 = (long long)lb * 256 * ORD_PT + threadIdx.x;
-    if (J.ord[w])
-        for (int u = 0; u < ORD_PT; ++u) {
-            const long long q = q0 + 256 * u;
-            if (q < J.nq[w]) atomicAdd(&h[order_bucket(J, w, q)], 1);
+    const int i0 = ends[0], ni = ends[1] - i0 + 1;
+#pragma unroll 4
+    for (int u = 0; u < ORD_PT; ++u) {
+        const int t = 256 * u + threadIdx.x;
+        const bool ok = t < nq;
+        int bucket = 0;
+        if (ok) {
+            const long long q = q0 + t;
+            const int i = i0 + last_le(b.qs + i0, ni, q);
+            const int j = b.j0[i] + (int)(q - b.qs[i]), P = a.bra[i], Q = a.ket[j];
+            quartets[q] = make_int2(P, Q);
+            kets[q] = a.ket_rec[j] | (P == Q ? 1u << 31 : 0u);
+            if (bk) {
+                bucket = order_bucket(a.pairs[P].n * (int)(a.ket_npcum[j + 1] - a.ket_npcum[j]));
+                bk[q] = (unsigned char)bucket;
+            }
         }
+        if (bk) {
+            const unsigned long long m = bucket_peers(bucket, ok);
+            if (ok && __ffsll((long long)m) - 1 == (int)(threadIdx.x & 63)) atomicAdd(&h[bucket], __popcll(m));
+        }
+    }
     __syncthreads();
-    if (threadIdx.x < ORD_NB && h[threadIdx.x]) atomicAdd(&cnt[jw * ORD_NB + threadIdx.x], h[threadIdx.x]);
+    if (bk && threadIdx.x < ORD_NB && h[threadIdx.x]) atomicAdd(&cnt[jw * ORD_NB + threadIdx.x], h[threadIdx.x]);
 }
 
 // cur[list][bucket] = exclusive scan of the list's bucket counts
@@ -239,33 +272,58 @@ __global__ void __launch_bounds__(64) list_order_scan_kernel(const int* cnt, int
 }
 
 // Every quartet takes a slot in its bucket: one global atomic per block and
-// bucket reserves the block's range, an LDS atomic gives the place in it.
+// bucket reserves the block's range, and within it the quartets keep their
+// list order (ranks within a wave by ballots, then a scan over the block's 64
+// groups of 64), so that neighbouring slots share a bra as often as they can.
+// With the buckets counted and kept by list_fill_batch_kernel the order costs
+// C14H30 36 us; counting and filling from the pairs' records took 130.
 __global__ void __launch_bounds__(256) list_order_fill_kernel(const ListJob* jobs, const ListBlocks blk, int* cur)
 {
-    __shared__ int h[ORD_NB], base[ORD_NB];
+    constexpr int NG = ORD_PT * 4, NSEG = 256 / ORD_NB, PER = NG / NSEG;
+    __shared__ int c[NG][ORD_NB], part[NSEG][ORD_NB], base[ORD_NB];
     int lb;
     const int jw = order_job_of(blk, lb), w = jw & 1;
     const ListJob& J = jobs[jw >> 1];
-    if (threadIdx.x < ORD_NB) h[threadIdx.x] = 0;
-    __syncthreads();
+    const unsigned char* const bk = J.bk[w];
+    int* const ord = J.ord[w];
+    const long long nq = J.nq[w];
+    if (!bk) return;
     const long long q0 = (long long)lb * 256 * ORD_PT + threadIdx.x;
-    int bk[ORD_PT], slot[ORD_PT];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int e = threadIdx.x; e < NG * ORD_NB; e += 256) ((int*)c)[e] = 0;
+    __syncthreads();
+    int bu[ORD_PT], rk[ORD_PT];
 #pragma unroll
     for (int u = 0; u < ORD_PT; ++u) {
-        const long long q = q0 + 256 * u;
-        bk[u] = -1;
-        slot[u] = 0;
-        if (J.ord[w] && q < J.nq[w]) {
-            bk[u] = order_bucket(J, w, q);
-            slot[u] = atomicAdd(&h[bk[u]], 1);
-        }
+        const bool ok = q0 + 256 * u < nq;
+        bu[u] = ok ? bk[q0 + 256 * u] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < ORD_PT; ++u) {
+        const unsigned long long m = bucket_peers(bu[u] & (ORD_NB - 1), bu[u] >= 0);
+        rk[u] = __popcll(m & ((1ULL << lane) - 1));
+        if (bu[u] >= 0 && rk[u] == 0) c[4 * u + wave][bu[u]] = __popcll(m);
     }
     __syncthreads();
-    if (threadIdx.x < ORD_NB && h[threadIdx.x]) base[threadIdx.x] = atomicAdd(&cur[jw * ORD_NB + threadIdx.x], h[threadIdx.x]);
+    const int k = threadIdx.x & (ORD_NB - 1), seg = threadIdx.x / ORD_NB;
+    int s = 0;
+    for (int g = 0; g < PER; ++g) s += c[seg * PER + g][k];
+    part[seg][k] = s;
+    __syncthreads();
+    int before = 0;
+    for (int g = 0; g < seg; ++g) before += part[g][k];
+    if (seg == NSEG - 1) base[k] = before + s ? atomicAdd(&cur[jw * ORD_NB + k], before + s) : 0;
+    __syncthreads();
+    int at = base[k] + before;
+    for (int g = 0; g < PER; ++g) {
+        const int n = c[seg * PER + g][k];
+        c[seg * PER + g][k] = at;
+        at += n;
+    }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < ORD_PT; ++u)
-        if (bk[u] >= 0) J.ord[w][base[bk[u]] + slot[u]] = (int)(q0 + 256 * u);
+        if (bu[u] >= 0) ord[c[4 * u + wave][bu[u]] + rk[u]] = (int)(q0 + 256 * u);
 }
 
 __global__ void __launch_bounds__(256) list_items_count_batch_kernel(const ListJob* jobs, const ListBlocks blk)
@@ -447,18 +505,17 @@ void list_scan_batch(const ScanJob* jobs, int n, hipStream_t st)
     if (n > 0) hipLaunchKernelGGL(list_scan_batch_kernel, dim3(n), dim3(1024), 0, st, jobs);
 }
 
-void list_fill_batch(const ListJob* jobs, const ListBlocks& blk, hipStream_t st)
-{
-    if (blk.n > 0 && blk.block0[blk.n] > 0)
-        hipLaunchKernelGGL(list_fill_batch_kernel, dim3(blk.block0[blk.n]), dim3(256), 0, st, jobs, blk);
-}
-
-void list_order_batch(const ListJob* jobs, const ListBlocks& blk, int* cnt, int* cur, hipStream_t st)
+void list_fill_batch(const ListJob* jobs, const ListBlocks& blk, int* cnt, hipStream_t st)
 {
     if (blk.n <= 0 || blk.block0[blk.n] <= 0) return;
     hipMemsetAsync(cnt, 0, sizeof(int) * ORD_NB * blk.n, st);
-    hipLaunchKernelGGL(list_order_count_kernel, dim3(blk.block0[blk.n]), dim3(256), 0, st, jobs, blk, cnt);
-    hipLaunchKernelGGL(list_order_scan_kernel, dim3(1), dim3(64), 0, st, (const int*)cnt, cur, blk.n);
+    hipLaunchKernelGGL(list_fill_batch_kernel, dim3(blk.block0[blk.n]), dim3(256), 0, st, jobs, blk, cnt);
+}
+
+void list_order_batch(const ListJob* jobs, const ListBlocks& blk, const int* cnt, int* cur, hipStream_t st)
+{
+    if (blk.n <= 0 || blk.block0[blk.n] <= 0) return;
+    hipLaunchKernelGGL(list_order_scan_kernel, dim3(1), dim3(64), 0, st, cnt, cur, blk.n);
     hipLaunchKernelGGL(list_order_fill_kernel, dim3(blk.block0[blk.n]), dim3(256), 0, st, jobs, blk, cur);
 }
 

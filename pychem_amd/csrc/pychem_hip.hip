@@ -413,6 +413,7 @@ struct pq_basis {
     const int* p_sorted[6] = {};
     const int* p_seg[6] = {};
     const long long* p_npcum[6] = {};
+    const unsigned* p_rec[6] = {};
     const double* p_sbound[6] = {};
     std::vector<char> hsortpack;
     std::vector<int> hseg[6], hsorted[6];    // host copies of what the device lists read
@@ -1129,7 +1130,7 @@ static int upload_sorted_pairs(pq_basis* b, hipStream_t st)
     }
     // one upload of every class's arrays (separate copies from pageable
     // memory cost ~20 us of host time each, 24 per plan); 256-byte sections
-    size_t off[6][4], total = 0;
+    size_t off[6][5], total = 0;
     auto take = [&](size_t bytes) {
         const size_t o = total;
         total += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
@@ -1140,6 +1141,7 @@ static int upload_sorted_pairs(pq_basis* b, hipStream_t st)
         off[X][1] = take(sizeof(int) * b->hseg[X].size());
         off[X][2] = take(sizeof(long long) * b->hnpcum[X].size());
         off[X][3] = take(sizeof(double) * b->hsbound[X].size());
+        off[X][4] = take(sizeof(unsigned) * b->hsorted[X].size());
     }
     if (b->d_sortpack.ensure(total)) return -1;
     // the host pack lives in the handle until the next plan, so the
@@ -1152,7 +1154,13 @@ static int upload_sorted_pairs(pq_basis* b, hipStream_t st)
         memcpy(h + off[X][1], b->hseg[X].data(), sizeof(int) * b->hseg[X].size());
         memcpy(h + off[X][2], b->hnpcum[X].data(), sizeof(long long) * b->hnpcum[X].size());
         memcpy(h + off[X][3], b->hsbound[X].data(), sizeof(double) * b->hsbound[X].size());
+        unsigned* rec = (unsigned*)(h + off[X][4]);
+        for (size_t k = 0; k < b->hsorted[X].size(); ++k) {
+            const PairHdr& p = b->pairs[b->hsorted[X][k]];
+            rec[k] = (unsigned)b->cart_off[p.s1] | ((unsigned)b->cart_off[p.s2] << 15) | (p.s1 == p.s2 ? 1u << 30 : 0u);
+        }
         b->p_sorted[X] = (const int*)(d + off[X][0]);
+        b->p_rec[X] = (const unsigned*)(d + off[X][4]);
         b->p_seg[X] = (const int*)(d + off[X][1]);
         b->p_npcum[X] = (const long long*)(d + off[X][2]);
         b->p_sbound[X] = (const double*)(d + off[X][3]);
@@ -1170,6 +1178,7 @@ static ListArgs list_args(const pq_basis* b, int c)
     a.bra_seg = b->p_seg[X];
     a.ket_seg = b->p_seg[Y];
     a.ket_npcum = b->p_npcum[Y];
+    a.ket_rec = b->p_rec[Y];
     a.bound = (const double*)b->d_bound.p;
     a.bra_bound = b->p_sbound[X];
     a.pairs = (const PairHdr*)b->d_pairs.p;
@@ -1363,12 +1372,16 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
         std::vector<ListJob> next = b->hjobs.back();   // the next phase's table: a new host copy
         b->hjobs.push_back(std::move(next));
     }
-    ListBlocks order_blocks = {};
-    order_blocks.n = 2 * ERI_NCLASS;
+    static const int order_env = [] {
+        const char* e = getenv("PQ_ERI_ORDER");
+        return e ? atoi(e) : 1;
+    }();
+    b->eri_order = order_env != 0;
+    ListBlocks fill_blocks = {};
+    fill_blocks.n = 2 * ERI_NCLASS;
+    if (b->d_order_cnt.ensure(sizeof(int) * 2 * ORD_NB * fill_blocks.n)) return -1;
     {
         std::vector<ListJob>& jobs = b->hjobs.back();
-        ListBlocks fb = {};
-        fb.n = 2 * ERI_NCLASS;
         for (int c = 0; c < ERI_NCLASS; ++c) {
             const int ncd = ncart_l(eri_class_table[c][2]) * ncart_l(eri_class_table[c][3]);
             for (int w = 0; w < 2; ++w) {
@@ -1382,26 +1395,28 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
                 jobs[c].q[w] = nullptr;
                 jobs[c].k[w] = nullptr;
                 jobs[c].ord[w] = nullptr;
+                jobs[c].bk[w] = nullptr;
                 if (s.nq) {
                     const size_t vb = (size_t)s.nq * s.ncomp * (w ? sizeof(float) : sizeof(double));
                     const size_t jb =
                         jk_tile_fits(b, c) ? sizeof(double) * (size_t)s.nq * jk_tile_table[c][2] * ncd : 0;
                     if (s.q.ensure(sizeof(int2) * s.nq) || s.vals.ensure(vb) ||
                         s.kets.ensure(sizeof(unsigned) * s.nq) || s.jkbuf.ensure(jb) ||
-                        (s.ncomp <= ORDER_MAX_NCOMP && s.order.ensure(sizeof(int) * s.nq)))
+                        (uses_order(b, s) && s.order.ensure((sizeof(int) + 1) * s.nq)))   // order, then buckets
                         return -1;
                     jobs[c].q[w] = (int2*)s.q.p;
                     jobs[c].k[w] = (unsigned*)s.kets.p;
-                    jobs[c].ord[w] = s.ncomp <= ORDER_MAX_NCOMP ? (int*)s.order.p : nullptr;
+                    if (uses_order(b, s)) {
+                        jobs[c].ord[w] = (int*)s.order.p;
+                        jobs[c].bk[w] = (unsigned char*)(jobs[c].ord[w] + s.nq);
+                    }
                 }
-                fb.block0[2 * c + w + 1] = fb.block0[2 * c + w] + (int)((nq + 255) / 256);
-                order_blocks.block0[2 * c + w + 1] =
-                    order_blocks.block0[2 * c + w] +
-                    (jobs[c].ord[w] ? (int)((nq + 256 * ORD_PT - 1) / (256 * ORD_PT)) : 0);
+                fill_blocks.block0[2 * c + w + 1] =
+                    fill_blocks.block0[2 * c + w] + (int)((nq + 256 * ORD_PT - 1) / (256 * ORD_PT));
             }
         }
         if (upload_jobs(jobs)) return -1;
-        list_fill_batch((const ListJob*)b->d_jobs.p, fb, st);
+        list_fill_batch((const ListJob*)b->d_jobs.p, fill_blocks, (int*)b->d_order_cnt.p, st);
     }
     {
         std::vector<ListJob> next = b->hjobs.back();   // the next phase's table: a new host copy
@@ -1461,18 +1476,10 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
         if (upload_jobs(jobs)) return -1;
         list_items_fill_batch((const ListJob*)b->d_jobs.p, tb, st);
         // the ERI kernels' quartet order (the table still holds every list's
-        // quartets and order buffer), queued after the plan's last host wait
-        static const int order_env = [] {
-            const char* e = getenv("PQ_ERI_ORDER");
-            return e ? atoi(e) : 1;
-        }();
-        b->eri_order = order_env != 0;
-        if (b->eri_order) {
-            const ListBlocks& ob = order_blocks;
-            if (b->d_order_cnt.ensure(sizeof(int) * 2 * ORD_NB * ob.n)) return -1;
-            int* cnt = (int*)b->d_order_cnt.p;
-            list_order_batch((const ListJob*)b->d_jobs.p, ob, cnt, cnt + ORD_NB * ob.n, st);
-        }
+        // buckets and order buffer), queued after the plan's last host wait
+        if (b->eri_order)
+            list_order_batch((const ListJob*)b->d_jobs.p, fill_blocks, (const int*)b->d_order_cnt.p,
+                             (int*)b->d_order_cnt.p + ORD_NB * fill_blocks.n, st);
     }
     HIPCHK(hipGetLastError());
     // table of the ket J reductions of every tiled list; every list's tiles
