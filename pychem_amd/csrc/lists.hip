@@ -214,8 +214,8 @@ __device__ __forceinline__ unsigned long long bucket_peers(int bucket, bool ok)
 // block's first and last quartet are searched once, each quartet's bra
 // between them, and what a quartet needs of its ket lies in ket order (one
 // search over all bras and three gathers, each behind the last, per quartet:
-X  Bucket and bucket counts are taken here, where both pairs'
-// primitive counts are at hand.
+// C14H30 122 us, 87 now).  Bucket and bucket counts are taken here, where both
+// pairs' primitive counts are at hand.
 __global__ void __launch_bounds__(256) list_fill_batch_kernel(const ListJob* jobs, const ListBlocks blk, int* cnt)
 {
     __shared__ int h[ORD_NB], ends[2];
