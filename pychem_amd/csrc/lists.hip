@@ -448,15 +448,16 @@ __global__ void __launch_bounds__(256) jket_reduce_kernel(const JredList L, cons
     jket_reduce_tile(L.a, L.b, L.w, L.jkbuf, L.nq, L.ntiles, L.ncd, L.n4, mols, J, L.tiles[t], cd);
 }
 
-// All lists in one launch: block -> list by the table's first-block offsets
-// (a handful of entries, scanned by every thread alike).
+// A run of the table's lists in one launch: block -> list by their first-block
+// offsets (a handful of entries, scanned by every thread alike).
 __global__ void __launch_bounds__(256) jket_reduce_all_kernel(const JredList* lists, int nlist, const MolInfo* mols,
                                                               double* J)
 {
     int c = 0;
-    while (c + 1 < nlist && lists[c + 1].block0 <= (long long)blockIdx.x) ++c;
+    const long long b = blockIdx.x + lists[0].block0;
+    while (c + 1 < nlist && lists[c + 1].block0 <= b) ++c;
     const JredList& L = lists[c];
-    const long long r = blockIdx.x - L.block0;
+    const long long r = b - L.block0;
     const int t = (int)(r % L.ntile), cd = (int)(r / L.ntile);
     jket_reduce_tile(L.a, L.b, L.w, L.jkbuf, L.nq, L.ntiles, L.ncd, L.n4, mols, J, L.tiles[t], cd);
 }

@@ -431,8 +431,10 @@ struct pq_basis {
     DevBuf d_jred;
     DevBuf d_jkgen;          // pq_jk_general scratch: symmetrised Dj, Dk^T, J2', K2'
     std::vector<JredList> hjred;
-    int njred = 0;
-    long long jred_blocks = 0;
+    // ket J reductions, in d_jred launch group by launch group: lists and
+    // blocks before group g
+    int jred_list0[JK_NGROUP + 1] = {};
+    long long jred_block0[JK_NGROUP + 1] = {};
     int nsorted[6] = {};
     DevBuf d_pairbase, d_pairtab;           // packed function pairs of the MP2 transform (ensure_pair_table)
     int npacked = 0;
@@ -1489,8 +1491,12 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
     std::vector<int4>& all = b->hjtiles_all;
     all.clear();
     long long blocks = 0;
-    for (int c = 0; c < ERI_NCLASS; ++c) {
-        if (!jk_tile_fits(b, c)) continue;
+    std::vector<int> tiled;   // classes by launch group
+    for (int g = 0; g < JK_NGROUP; ++g)
+        for (int c = 0; c < ERI_NCLASS; ++c)
+            if (jk_group_table[c] == g && jk_tile_fits(b, c)) tiled.push_back(c);
+    for (int g = 0; g <= JK_NGROUP; ++g) b->jred_list0[g] = b->jred_block0[g] = 0;
+    for (int c : tiled) {
         const int n3 = ncart_l(eri_class_table[c][2]), n4 = ncart_l(eri_class_table[c][3]);
         for (int w = 0; w < 2; ++w) {
             EriClassStore& s = w ? b->store32[c] : b->store64[c];
@@ -1509,14 +1515,17 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
             blocks += (long long)L.ntile * L.ncd;
             jr.push_back(L);
         }
+        for (int g = jk_group_table[c] + 1; g <= JK_NGROUP; ++g) {
+            b->jred_list0[g] = (int)jr.size();
+            b->jred_block0[g] = blocks;
+        }
     }
     if (b->d_jtiles.ensure(sizeof(int4) * std::max<size_t>(1, all.size()))) return -1;
     if (!all.empty())
         HIPCHK(hipMemcpyAsync(b->d_jtiles.p, all.data(), sizeof(int4) * all.size(), hipMemcpyHostToDevice, st));
     {
         size_t k = 0;
-        for (int c = 0; c < ERI_NCLASS; ++c) {
-            if (!jk_tile_fits(b, c)) continue;
+        for (int c : tiled) {
             for (int w = 0; w < 2; ++w) {
                 EriClassStore& s = w ? b->store32[c] : b->store64[c];
                 if (!s.nq) continue;
@@ -1527,8 +1536,6 @@ extern "C" int pq_eri_plan(pq_basis* b, double threshold, double fp32_threshold,
         }
     }
     if (blocks > 0x7fffffffLL) return fail("pq_eri_plan: ket J reduction grid too large");
-    b->njred = (int)jr.size();
-    b->jred_blocks = blocks;
     if (b->d_jred.ensure(sizeof(JredList) * std::max<size_t>(1, jr.size()))) return -1;
     b->hjred = std::move(jr);   // kept in the handle: no wait for the upload
     if (!b->hjred.empty())
@@ -1882,8 +1889,14 @@ static int jk_launch_class(pq_basis* b, int c, const double* Dj, const double* D
 // class's reduction launched behind its digestion on the side stream instead
 // was slower: the many small reduction launches queue behind the digestion
 // kernels.)
+static void jk_reduce_groups(pq_basis* b, int g0, int g1, double* J, hipStream_t st)
+{
+    jket_reduce_all((const JredList*)b->d_jred.p + b->jred_list0[g0], b->jred_list0[g1] - b->jred_list0[g0],
+                    b->jred_block0[g1] - b->jred_block0[g0], (const MolInfo*)b->d_mols.p, J, st);
+}
+
 static int jk_digest_all(pq_basis* b, const double* Dj, const double* Dk, double* J, double* K, hipStream_t st,
-                         bool single_stream)
+                         bool single_stream, bool reduce)
 {
     // classes by stored bytes per block, so that the longest blocks start first
     int order[ERI_NCLASS], nc = 0;
@@ -1934,6 +1947,11 @@ static int jk_digest_all(pq_basis* b, const double* Dj, const double* Dk, double
     // digestions, 458 / 441; C10H22, 0.55 GB, 309 / 315; C14H30 613 / 654).
     const bool small = gb[0] + gb[1] + gb[2] + gb[3] < 400e6;
     const int ns = single_stream || small ? 1 : std::min(n, std::min(4, std::max(1, b->jk_nstreams)));
+    // From 1 GB on a group's ket J values are summed behind it on its stream,
+    // while other groups still run and its values may still lie in the
+    // Infinity Cache (C20H42, 2.9 GB: 1143 us with one launch for all behind
+    // the join, 1117 so); below, the launches cost more (C10H22 285 / 291).
+    const bool behind = ns > 1 && gb[0] + gb[1] + gb[2] + gb[3] >= 1e9;
     if (ns > 1) {
         if (ensure_jk_streams(b)) return -1;
         HIPCHK(hipEventRecord(b->ev_fork, st));
@@ -1946,12 +1964,15 @@ static int jk_digest_all(pq_basis* b, const double* Dj, const double* Dk, double
         for (int t = 1; t < ns; ++t)
             if (load[t] < load[k]) k = t;
         load[k] += gb[g];
-        if (jk_group_launch(b, g, in[g], ng[g], 3, Dj, Dk, J, K, k > 0 ? b->jk_side[k - 1] : st)) return -1;
+        hipStream_t sk = k > 0 ? b->jk_side[k - 1] : st;
+        if (jk_group_launch(b, g, in[g], ng[g], 3, Dj, Dk, J, K, sk)) return -1;
+        if (reduce && behind) jk_reduce_groups(b, g, g + 1, J, sk);
     }
     for (int k = 1; k < ns; ++k) {
         HIPCHK(hipEventRecord(b->ev_join[k - 1], b->jk_side[k - 1]));
         HIPCHK(hipStreamWaitEvent(st, b->ev_join[k - 1], 0));
     }
+    if (reduce && !behind) jk_reduce_groups(b, 0, JK_NGROUP, J, st);
     jk_clock_set(b, 1, st);
     return 0;
 }
@@ -1968,8 +1989,7 @@ static int jk_launch_all(pq_basis* b, const double* Dj, const double* Dk, double
 {
     const MolInfo* dm = (const MolInfo*)b->d_mols.p;
     jk_zero(b, J, K, st);
-    if (jk_digest_all(b, Dj, Dk, J, K, st, false)) return -1;
-    jket_reduce_all((const JredList*)b->d_jred.p, b->njred, b->jred_blocks, dm, J, st);
+    if (jk_digest_all(b, Dj, Dk, J, K, st, false, true)) return -1;
     int gx = (int)((b->nmax * (long long)b->nmax + 255) / 256);
     gx = gx < 1 ? 1 : (gx > 64 ? 64 : gx);
     hipLaunchKernelGGL(jk_finish_kernel, dim3(gx, b->nmol), dim3(256), 0, st, J, K, dm);
@@ -2057,9 +2077,8 @@ static int jk_general_run(pq_basis* b, const double* Dj, const double* Dk, doubl
         double* Kp = pass ? K : K2;
         const double* Dkp = pass ? (const double*)DkT : Dk;
         jk_zero(b, Jp, Kp, st);
-        if (jk_digest_all(b, Ds, Dkp, Jp, Kp, st, single_stream)) return -1;
+        if (jk_digest_all(b, Ds, Dkp, Jp, Kp, st, single_stream, pass == 1)) return -1;   // J is the second pass's
     }
-    jket_reduce_all((const JredList*)b->d_jred.p, b->njred, b->jred_blocks, dm, J, st);
     hipLaunchKernelGGL(jk_general_finish_kernel, dim3(gx, b->nmol), dim3(256), 0, st, J, K, K2, dm);
     HIPCHK(hipGetLastError());
     return 0;

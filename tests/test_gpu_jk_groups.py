@@ -115,3 +115,30 @@ def test_rows_beyond_64_kib_of_lds(gpu):
         assert (blk - K1).abs().max().item() < 1e-10 * K1.abs().max().item()
     for e in es:
         e.close()
+
+
+@pytest.mark.parametrize("fp32", [0.0, 1e-5])
+def test_reductions_behind_each_group(gpu, fp32):
+    """Above 1 GB of stored integrals the ket sums of a group run behind it on
+    its own stream: four streams against one.  A term of J_ab is at most
+    Q_ab Q_cd |D_cd| (Schwarz), in any order of n^2 additions."""
+    import torch
+    from pychem_amd import _lib
+    from pychem_amd.engine import Engine
+    m = structures.Molecule(geometry.alkane(16, 0.05, 5), basis="6-31G*", cartesian_l=[2], multiplicity=1)
+    e = Engine(m)
+    e.build_eri(1e-8, fp32)
+    n = e.ncart
+    assert sum((s["nq64"] * 8 + s["nq32"] * 4) * s["ncomp"] for s in e.stats()) > 1e9 or fp32
+    D = np.random.default_rng(9).normal(size=(2, n, n))
+    D = torch.as_tensor(D + D.transpose(0, 2, 1), device="cuda")
+    L = _lib.lib()
+    out = {}
+    for ns in (1, 4):
+        _lib.check(L.pq_jk_set_streams(e.h, ns), "pq_jk_set_streams")
+        out[ns] = _jk(e, D)
+    Q = e.schwarz()
+    tol = 4 * (n * n + 16) * U * Q.max() * Q.sum() * 36 * float(D.abs().max())
+    for a, b in zip(out[1], out[4]):
+        assert np.abs(a - b).max() <= tol
+    assert np.abs(out[1][0]).max() > 1e3 * tol
