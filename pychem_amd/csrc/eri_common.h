@@ -33,7 +33,7 @@ struct MolInfo {
 // 96 bytes, so that every record starts on a 16-byte boundary.
 template <typename real>
 struct PrimPair {
-    real Px, Py, Pz, PAx, PAy, PAz, p, inv2p, K, beta, Ks, pad;
+    real Px, Py, Pz, p, Ks, PAx, PAy, PAz, inv2p, K, beta, pad;
 };
 
 // Constant address space: a load through such a pointer at a wave-uniform

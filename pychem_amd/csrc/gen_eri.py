@@ -273,7 +273,7 @@ def split_groups(la, lc, na, nc):
 
 # Occupancy floor per class kernel (waves per SIMD, the second argument of
 # __launch_bounds__); 1 leaves the register count to the compiler.
-MINW = {"2020": 2, "2220": 2}   # measured on C20H42/6-31G*: 0.087 -> 0.067 ms, 0.085 -> 0.064 ms
+MINW = {"2020": 2, "2220": 2, "2110": 2}   # measured on C20H42/6-31G*: 0.087 -> 0.067 ms, 0.085 -> 0.064 ms
 
 # classes with at most this many VRR/contraction lines per primitive quartet
 # get the scalar-load path for wave-uniform bras
