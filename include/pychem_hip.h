@@ -337,6 +337,34 @@ int pq_eigh_batched(const double* A_dev, int batch, int n, double* w_dev, double
 int pq_purify_batched(const double* M_dev, const int* nocc_dev, int batch, int m, double tol, int max_steps,
                       double* P_dev, int* steps_dev, void* stream);
 
+/* The batched SCF between its matrix products, one workgroup per molecule.
+ * Matrices [batch][m][m] (m <= 30000), molecule b's in the leading n[b] x
+ * n[b] corner; packed arrays hold the n[b] x n[b] blocks from element base[b]
+ * on (base, n: device arrays of batch).  All pointers are device pointers.
+ * pack: D <- Dn where !done (Dn NULL: unchanged), Dj = 2 D and Dk = D packed.
+ * fock: F = H + J + K, J and K packed.
+ * test: E[b] = sum D (H + F) + enuc[b] and iters[b] = it of the molecules not
+ *   done; done[b] (and newly[b] = 1) once, for it > 1, E moved by less than
+ *   conv and max |R| <= rtol.  flags: [0] set when any is newly done, [1]
+ *   counts those not done (both zeroed by the caller).
+ * diis: ring slot `newest` of Fbuf, Rbuf [batch][slots][m][m] takes F and R,
+ *   G [batch][slots][slots] their products with the last k slots, and Fx is
+ *   Pulay's combination of the last k Fock matrices (F itself for k = 1).
+ *   flags[2] counts singular systems.  work: pq_batch_diis_work doubles.
+ * lift: M += diag(dropped t), t one above the Gershgorin bound of M (at least
+ *   1), dropped [batch][m]. */
+int pq_batch_pack(int batch, int m, const long long* base, const long long* n, double* D, const double* Dn,
+                  const unsigned char* done, double* Dj, double* Dk, void* stream);
+int pq_batch_fock(int batch, int m, const long long* base, const long long* n, const double* H, const double* J,
+                  const double* K, double* F, void* stream);
+int pq_batch_test(int batch, int m, const long long* n, const double* D, const double* H, const double* F,
+                  const double* R, const double* enuc, double conv, double rtol, int it, double* E, long long* iters,
+                  unsigned char* done, unsigned char* newly, int* flags, void* stream);
+long long pq_batch_diis_work(int batch, int k);
+int pq_batch_diis(int batch, int m, const double* F, const double* R, double* Fbuf, double* Rbuf, double* G, int slots,
+                  int newest, int k, double* Fx, double* work, int* flags, void* stream);
+int pq_batch_lift(int batch, int m, double* M, const double* dropped, void* stream);
+
 /* MP2 energy sum over ovov [o1][v1][o2][v2] with D = e_i + e_j - e_a - e_b:
  * mode 0 closed shell sum v(2v - (ib|ja))/D; mode 1 same spin
  * 1/4 sum ((ia|jb) - (ib|ja))^2 / D; mode 2 opposite spin sum v^2 / D

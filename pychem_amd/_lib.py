@@ -93,6 +93,12 @@ SIGNATURES = {
     "pq_eigh_refine_work": (ctypes.c_longlong, [c_int]),
     "pq_eigh_batched": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "pq_purify_batched": (c_int, [c_void_p, c_void_p, c_int, c_int, c_double, c_int, c_void_p, c_void_p, c_void_p]),
+    "pq_batch_pack": (c_int, [c_int, c_int] + [c_void_p] * 8),
+    "pq_batch_fock": (c_int, [c_int, c_int] + [c_void_p] * 7),
+    "pq_batch_test": (c_int, [c_int, c_int] + [c_void_p] * 6 + [c_double, c_double, c_int] + [c_void_p] * 6),
+    "pq_batch_diis_work": (ctypes.c_longlong, [c_int, c_int]),
+    "pq_batch_diis": (c_int, [c_int, c_int] + [c_void_p] * 5 + [c_int, c_int, c_int] + [c_void_p] * 4),
+    "pq_batch_lift": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "pq_eigh_refine": (c_int, [c_void_p, c_void_p, c_int, c_int, c_double, c_void_p, c_void_p, P_double, c_void_p]),
     "pq_mp2_energy": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                               c_int, P_double, c_void_p]),

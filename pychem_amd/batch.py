@@ -73,6 +73,7 @@ class BatchEngine:
         nrow = torch.repeat_interleave(nn, sizes, **rep)
         self.pidx = mol * nm * nm + torch.div(k, nrow, rounding_mode="floor") * nm + k % nrow
         self.n_dev = nn
+        self.base_dev = torch.cumsum(sizes, 0) - sizes
         self.graph = False
 
     def close(self):
@@ -127,6 +128,22 @@ class BatchEngine:
 
     def jk_replay(self):
         check(_lib.lib().pq_jk_graph_launch(self.h, _stream()), "pq_jk_graph_launch")
+
+    # the SCF's steps between its matrix products, one launch each, on padded
+    # matrices [nmol, nmax, nmax] (scf_batch.hip)
+    def _call(self, name, *args):
+        check(getattr(_lib.lib(), name)(self.nmol, self.nmax, *args, _stream()), name)
+
+    def pack(self, D, Dn=None, done=None):
+        """D <- Dn where not done; the J/K inputs Dj = 2 D and Dk = D."""
+        self._call("pq_batch_pack", _ptr(self.base_dev), _ptr(self.n_dev), _ptr(D),
+                   None if Dn is None else _ptr(Dn), None if done is None else _ptr(done), _ptr(self.Dj), _ptr(self.Dk))
+
+    def fock(self, H):
+        """H + J + K of the last J/K build."""
+        F = torch.empty_like(H)
+        self._call("pq_batch_fock", _ptr(self.base_dev), _ptr(self.n_dev), _ptr(H), _ptr(self.J), _ptr(self.K), _ptr(F))
+        return F
 
     def jk_direct(self):
         check(_lib.lib().pq_jk(self.h, _ptr(self.Dj), _ptr(self.Dk), _ptr(self.J), _ptr(self.K), _stream()), "pq_jk")
@@ -185,7 +202,7 @@ def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_grap
     nocc_h = np.array([m.NAlphaElectrons for m in mols])
     enuc_h = _nuclear_batch(eng)
     D_h = _sad_padded(eng, mols, host=True) if guess == "SAD" else None
-    nocc = torch.as_tensor(nocc_h, device=dev)
+    nocc = torch.as_tensor(nocc_h, device=dev).to(torch.int32)
     enuc = torch.as_tensor(enuc_h, dtype=torch.float64, device=dev)
     if guess == "SAD":
         D = 0.5 * torch.as_tensor(D_h).to(dev)
@@ -213,24 +230,27 @@ def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_grap
     t_setup = time.perf_counter() - t_start
     E = torch.zeros(B, dtype=torch.float64, device=dev)
     done = torch.zeros(B, dtype=torch.bool, device=dev)
+    newly = torch.zeros_like(done)
     iters = torch.zeros(B, dtype=torch.long, device=dev)
     latency = np.full(B, np.nan)
-    # DIIS history in slot buffers (no per-iteration stacking): the stored
-    # Fock matrices and residuals, their Gram matrix updated by one batched
-    # product per iteration, the active slots oldest first
+    # DIIS history in a ring of slots: the stored Fock matrices and residuals
+    # and their Gram matrix, the last k slots active
     S_ = diis_size + 1
     Fbuf = torch.zeros((B, S_, nm, nm), dtype=torch.float64, device=dev)
     Rbuf = torch.zeros_like(Fbuf)
     G = torch.zeros((B, S_, S_), dtype=torch.float64, device=dev)
-    slots = []
+    work = None
+    # per cycle: any newly converged, molecules not converged, singular systems
+    flags = torch.zeros((max(maxiter, 0) + 1, 3), dtype=torch.int32, device=dev)
+    D, Hp, Dn = D.contiguous(), Hp.contiguous(), None
     for it in range(1, maxiter + 1):
-        eng.to_packed(2.0 * D, out=eng.Dj)
-        eng.to_packed(D, out=eng.Dk)
+        eng.pack(D, Dn, done)
+        Dn = None
         if use_graph:
             eng.jk_replay()
         else:
             eng.jk_direct()
-        F = Hp + eng.to_padded(eng.J) + eng.to_padded(eng.K)
+        F = eng.fock(Hp)
         # Pulay DIIS on X^T (S D F - F D S) X, batched
         A = Sp @ D @ F
         R = X.transpose(1, 2) @ (A - A.transpose(1, 2)) @ X
@@ -238,48 +258,28 @@ def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_grap
         # matrix (the single-molecule device loop's test): |dE| < conv counts
         # once the orbital gradient has settled too, and the molecule keeps
         # the density whose energy passed
-        Ev = ((D * (Hp + F)) * vmask).sum((1, 2)) + enuc
-        rmax = R.abs().amax((1, 2))
-        newly = (~done) & ((Ev - E).abs() < conv) & (rmax <= conv ** 0.5) & (it > 1)
-        E = torch.where(done, E, Ev)
-        iters = torch.where(done, iters, torch.full_like(iters, it))
-        done_next = done | newly
-        any_new, all_done = torch.stack([newly.any(), done_next.all()]).tolist()   # one host wait per iteration
+        eng._call("pq_batch_test", _ptr(eng.n_dev), _ptr(D), _ptr(Hp), _ptr(F), _ptr(R), _ptr(enuc), float(conv),
+                  float(conv) ** 0.5, it, _ptr(E), _ptr(iters), _ptr(done), _ptr(newly), _ptr(flags[it]))
+        # one host wait per iteration (the singular systems are the last cycle's)
+        (_, _, singular), (any_new, not_done, _) = flags[it - 1:it + 1].tolist()
+        if singular:
+            raise torch.linalg.LinAlgError("rhf_batch: singular DIIS system")
         if any_new:
             tnow = time.perf_counter() - t_start
             for m in torch.nonzero(newly).flatten().tolist():
                 latency[m] = tnow
-        done = done_next
-        if all_done:
+        if not not_done:
             break
-        free = next(t for t in range(S_) if t not in slots)
-        Fbuf[:, free] = F
-        Rbuf[:, free] = R
-        g = torch.bmm(Rbuf.view(B, S_, nm * nm), R.reshape(B, nm * nm, 1))[:, :, 0]   # [B, S_]
-        G[:, free, :] = g
-        G[:, :, free] = g
-        slots.append(free)
-        if len(slots) > diis_size:
-            slots.pop(0)
-        k = len(slots)
-        if k >= 2:
-            sl = torch.as_tensor(slots, device=dev)
-            Bm = G.index_select(1, sl).index_select(2, sl)                 # [B, k, k]
-            A = torch.full((B, k + 1, k + 1), -1.0, dtype=torch.float64, device=dev)
-            A[:, :k, :k] = Bm
-            A[:, k, k] = 0.0
-            # tiny ridge keeps the bordered system regular for converged molecules
-            A[:, :k, :k] += torch.diag_embed((1e-14 * Bm.diagonal(dim1=1, dim2=2).mean(1, keepdim=True)
-                                              + 1e-300).expand(B, k))
-            rhs = torch.zeros((B, k + 1, 1), dtype=torch.float64, device=dev)
-            rhs[:, k, 0] = -1.0
-            c = torch.linalg.solve(A, rhs)[:, :k, 0]                     # [B, k]
-            cf = torch.zeros((B, S_), dtype=torch.float64, device=dev)
-            cf[:, sl] = c
-            Fx = torch.bmm(cf[:, None, :], Fbuf.view(B, S_, nm * nm)).view(B, nm, nm)
-        else:
-            Fx = F
-        Dn = _density(X, Fx, dropped, nocc)
+        k = max(1, min(it, diis_size))
+        if work is None or k > 64:
+            work = torch.empty(max(1, _lib.lib().pq_batch_diis_work(B, k)), dtype=torch.float64, device=dev)
+        Fx = torch.empty_like(F)
+        eng._call("pq_batch_diis", _ptr(F), _ptr(R), _ptr(Fbuf), _ptr(Rbuf), _ptr(G), S_, (it - 1) % S_, k, _ptr(Fx),
+                  _ptr(work), _ptr(flags[it]))
+        Dn = _density(X, Fx, dropped, nocc).contiguous()
+    if Dn is not None:   # not every molecule converged
+        if flags[it, 2].item():
+            raise torch.linalg.LinAlgError("rhf_batch: singular DIIS system")
         D = torch.where(done[:, None, None], D, Dn)
     torch.cuda.synchronize()
     total = time.perf_counter() - t_start
@@ -301,10 +301,8 @@ def _density(X, F, dropped, nocc):
     so that they stay empty."""
     from .engine import EIGH_BATCHED_MAXN, purify_batched as purify_lib
     from .hartree_fock import purify_batched
-    M = X.transpose(1, 2) @ F @ X
-    diag = M.diagonal(dim1=1, dim2=2)
-    top = (diag + M.abs().sum(2) - diag.abs()).max(1).values.clamp_min(0.0) + 1.0
-    M = M + torch.diag_embed(dropped * top[:, None])
+    M = (X.transpose(1, 2) @ F @ X).contiguous()
+    check(_lib.lib().pq_batch_lift(M.shape[0], M.shape[1], _ptr(M), _ptr(dropped), _stream()), "pq_batch_lift")
     if M.shape[1] <= EIGH_BATCHED_MAXN:
         P, _ = purify_lib(M, nocc)
     else:
