@@ -158,106 +158,147 @@ extern "C" int pq_eigh_batched(const double* A, int batch, int n, double* w, dou
 // ---------------------------------------------------------------------------
 // Density projectors of many small Fock matrices at once (the batched SCF):
 // trace-correcting purification (TC2: Niklasson, Phys. Rev. B 66, 155115
-// (2002)) with one workgroup per matrix, X and X^2 in LDS, padded with zeros
-// to mp = m rounded up to 16 in both dimensions.  X0 = (e_max - M) / (e_max -
-// e_min) with Gershgorin bounds; each step forms X^2 on the FP64 matrix cores
-// (X symmetric: (X^2)_ij = sum_k X_ki X_kj, both operands read along row k of
-// X; wave w owns the 16-row blocks w, w + 4, ... and every 16-column block of
-// them; v_mfma_f64_16x16x4f64 step t gives lane l the k = 4 t + l / 16, its
-// A element X[k][i0 + l % 16] and B element X[k][j0 + l % 16], and result
-// register r of lane l is (X^2)[i0 + 4 r + l / 16][j0 + l % 16]), then keeps
-// X^2 or 2X - X^2, whichever trace is nearer nocc; once tr(X - X^2) < tol one
-// more step is taken.  P = (X + X^T) / 2; steps[b] = the steps taken
-// (max_steps + 1 when the tolerance was never met).
-#define PURIFY_MAXNB ((EIGH_MAXN + 15) / 16)
-__global__ void __launch_bounds__(256) purify_small_kernel(const double* __restrict__ M, const int* __restrict__ nocc,
-                                                           int m, double tol, int max_steps, double* __restrict__ P,
-                                                           int* __restrict__ steps)
+// (2002)) with one workgroup per matrix, X in LDS.  X0 = (e_max - M) / (e_max
+// - e_min) with Gershgorin bounds; each step forms X^2 on the FP64 matrix
+// cores (X symmetric: (X^2)_ij = sum_k X_ki X_kj, both operands read along row
+// k of X; wave w owns the 16 x 16 tiles w, w + 8, ...; v_mfma_f64_16x16x4f64
+// step t gives lane l the k = 4 t + l / 16, its A element X[k][i0 + l % 16]
+// and B element X[k][j0 + l % 16], and result register r of lane l is
+// (X^2)[i0 + 4 r + l / 16][j0 + l % 16]), then keeps X^2 or 2X - X^2,
+// whichever trace is nearer nocc; once tr(X - X^2) < tol one more step is
+// taken.  P = (X + X^T) / 2; steps[b] = the steps taken (max_steps + 1 when
+// the tolerance was never met).
+//
+// A batch is padded to its largest molecule: on average a third of the rows
+// belong to a molecule, the rest couple to nothing.  Only the leading block up
+// to the last coupled row, me rounded up to 16, is multiplied; the diagonal
+// beyond it is squared element by element, which is the same arithmetic.  X^2
+// stays in registers until the traces have chosen, so that X is the only
+// matrix in LDS and several workgroups share a CU.  512 molecules of 7 to 61
+// functions: 228 us, 338 with every row multiplied and X^2 in LDS.
+#define PURIFY_W 8
+#define PURIFY_MAXT ((EIGH_MAXN + 15) / 16 * ((EIGH_MAXN + 15) / 16))
+__global__ void __launch_bounds__(64 * PURIFY_W) purify_small_kernel(const double* __restrict__ M,
+                                                                     const int* __restrict__ nocc, int m, double tol,
+                                                                     int max_steps, double* __restrict__ P,
+                                                                     int* __restrict__ steps)
 {
     typedef double pd4 __attribute__((ext_vector_type(4)));
+    constexpr int NT = (PURIFY_MAXT + PURIFY_W - 1) / PURIFY_W;   // tiles of a wave
     extern __shared__ double sh[];
-    const int mp = (m + 15) & ~15;
-    double* X = sh;             // mp x mp
-    double* X2 = sh + mp * mp;  // mp x mp
-    __shared__ double red[16];
-    const int tid = threadIdx.x, nt = blockDim.x;
+    __shared__ double red[2][2][PURIFY_W], d[EIGH_MAXN];
+    __shared__ int s_me;
+    const int tid = threadIdx.x, nt = 64 * PURIFY_W;
     const int wave = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
     const size_t off = (size_t)blockIdx.x * m * m;
-    for (int i = tid; i < mp * mp; i += nt) {
-        const int r = i / mp, c = i - r * mp;
-        X2[i] = (r < m && c < m) ? M[off + (size_t)r * m + c] : 0.0;
-    }
+    if (tid == 0) s_me = 0;
     __syncthreads();
-    // Gershgorin bounds (row i: M_ii -/+ sum_{j != i} |M_ij|)
+    // Gershgorin bounds (row i: M_ii -/+ sum_{j != i} |M_ij|) and the last
+    // row with a coupling
     double lo = 1e300, hi = -1e300;
-    for (int r = tid; r < m; r += nt) {
+    int me = 0;
+    for (int r = wave; r < m; r += PURIFY_W) {
         double rad = 0.0;
-        for (int c = 0; c < m; ++c)
-            if (c != r) rad += fabs(X2[r * mp + c]);
-        lo = fmin(lo, X2[r * mp + r] - rad);
-        hi = fmax(hi, X2[r * mp + r] + rad);
-    }
+        for (int c = lane; c < m; c += 64) {
+            const double v = M[off + (size_t)r * m + c];
+            if (c == r) continue;
+            rad += fabs(v);
+            if (v != 0.0) me = max(me, max(r, c) + 1);
+        }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        lo = fmin(lo, __shfl_xor(lo, o, 64));
-        hi = fmax(hi, __shfl_xor(hi, o, 64));
+        for (int o = 32; o > 0; o >>= 1) rad += __shfl_xor(rad, o, 64);
+        const double v = M[off + (size_t)r * m + r];
+        lo = fmin(lo, v - rad);
+        hi = fmax(hi, v + rad);
     }
-    if ((tid & 63) == 0) {
-        red[tid >> 6] = lo;
-        red[8 + (tid >> 6)] = hi;
+    if (me) atomicMax(&s_me, me);
+    if (lane == 0) {
+        red[0][0][wave] = lo;
+        red[0][1][wave] = hi;
     }
     __syncthreads();
-    double emin = red[0], emax = red[8];
-    for (int w = 1; w < (int)(nt >> 6); ++w) {
-        emin = fmin(emin, red[w]);
-        emax = fmax(emax, red[8 + w]);
+    double emin = red[0][0][0], emax = red[0][1][0];
+    for (int w = 1; w < PURIFY_W; ++w) {
+        emin = fmin(emin, red[0][0][w]);
+        emax = fmax(emax, red[0][1][w]);
     }
+    me = s_me;
+    const int nb = (me + 15) / 16, mp = 16 * nb, ntile = nb * nb, mx = min(m, mp);
+    double* const X = sh;   // mp x mp
     const double inv = 1.0 / (emax - emin);
     for (int i = tid; i < mp * mp; i += nt) {
         const int r = i / mp, c = i - r * mp;
-        X[i] = (r < m && c < m) ? ((r == c ? emax : 0.0) - X2[i]) * inv : 0.0;
+        X[i] = (r < m && c < m) ? ((r == c ? emax : 0.0) - M[off + (size_t)r * m + c]) * inv : 0.0;
     }
+    for (int i = mx + tid; i < m; i += nt) d[i] = (emax - M[off + (size_t)i * m + i]) * inv;
     __syncthreads();
     const double nf = (double)nocc[blockIdx.x];
-    const int nb = mp / 16;
     int k = 0;
     bool last = false;
     for (; k < max_steps; ++k) {
-        for (int ib = wave; ib < nb; ib += (int)(nt >> 6)) {
-            const int i0 = 16 * ib;
-            pd4 acc[PURIFY_MAXNB];
-#pragma unroll
-            for (int jb = 0; jb < PURIFY_MAXNB; ++jb) acc[jb] = (pd4){0.0, 0.0, 0.0, 0.0};
-            for (int t = 0; t < mp / 4; ++t) {
-                const double* row = X + (4 * t + lq) * mp;
-                const double a = row[i0 + li];
-#pragma unroll
-                for (int jb = 0; jb < PURIFY_MAXNB; ++jb)
-                    if (jb < nb) acc[jb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, row[16 * jb + li], acc[jb], 0, 0, 0);
-            }
-#pragma unroll
-            for (int jb = 0; jb < PURIFY_MAXNB; ++jb)
-                if (jb < nb)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) X2[(i0 + 4 * r + lq) * mp + 16 * jb + li] = acc[jb][r];
-        }
-        __syncthreads();
+        pd4 acc[NT];
         double t1 = 0.0, t2 = 0.0;
-        for (int i = tid; i < m; i += nt) {
-            t1 += X[i * mp + i];
-            t2 += X2[i * mp + i];
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int t = wave + PURIFY_W * u;
+            if (t >= ntile) break;
+            const int i0 = 16 * (t / nb), j0 = 16 * (t % nb);
+            pd4 a = (pd4){0.0, 0.0, 0.0, 0.0};
+            const double* pa = X + lq * mp + i0 + li;
+            const double* pb = X + lq * mp + j0 + li;
+#pragma unroll 4
+            for (int q = 0; q < mp / 4; ++q)
+                a = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[4 * q * mp], pb[4 * q * mp], a, 0, 0, 0);
+            acc[u] = a;
+            if (i0 == j0) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (4 * r + lq == li) {
+                        t1 += X[(i0 + li) * mp + i0 + li];
+                        t2 += a[r];
+                    }
+            }
         }
-        t1 = eigh_block_sum(t1, red);
-        t2 = eigh_block_sum(t2, red);
+        for (int i = mx + tid; i < m; i += nt) {
+            t1 += d[i];
+            t2 += d[i] * d[i];
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            t1 += __shfl_xor(t1, o, 64);
+            t2 += __shfl_xor(t2, o, 64);
+        }
+        if (lane == 0) {
+            red[k & 1][0][wave] = t1;
+            red[k & 1][1][wave] = t2;
+        }
+        __syncthreads();   // every wave has read X
+        t1 = t2 = 0.0;
+#pragma unroll
+        for (int w = 0; w < PURIFY_W; ++w) {
+            t1 += red[k & 1][0][w];
+            t2 += red[k & 1][1][w];
+        }
         const bool up = fabs(t2 - nf) < fabs(2.0 * t1 - t2 - nf);
-        for (int i = tid; i < mp * mp; i += nt) X[i] = up ? X2[i] : 2.0 * X[i] - X2[i];
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int t = wave + PURIFY_W * u;
+            if (t >= ntile) break;
+            const int i0 = 16 * (t / nb), j0 = 16 * (t % nb);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double* x = X + (i0 + 4 * r + lq) * mp + j0 + li;
+                *x = up ? acc[u][r] : 2.0 * *x - acc[u][r];
+            }
+        }
+        for (int i = mx + tid; i < m; i += nt) d[i] = up ? d[i] * d[i] : 2.0 * d[i] - d[i] * d[i];
         __syncthreads();
         if (last) break;
         if (t1 - t2 < tol) last = true;
     }
     for (int i = tid; i < m * m; i += nt) {
         const int r = i / m, c = i - r * m;
-        P[off + i] = 0.5 * (X[r * mp + c] + X[c * mp + r]);
+        P[off + i] = r < mx && c < mx ? 0.5 * (X[r * mp + c] + X[c * mp + r]) : (r == c ? d[r] : 0.0);
     }
     if (tid == 0) steps[blockIdx.x] = last ? k + 1 : max_steps + 1;
 }
@@ -272,16 +313,16 @@ extern "C" int pq_purify_batched(const double* M, const int* nocc, int batch, in
                              std::to_string(EIGH_MAXN)).c_str());
     if (batch == 0) return 0;
     const int mp = (m + 15) & ~15;
-    const size_t lds = sizeof(double) * 2 * (size_t)mp * mp;
+    const size_t lds = sizeof(double) * (size_t)mp * mp;
     static bool attr = false;
     if (!attr) {
-        const int mpmax = (EIGH_MAXN + 15) & ~15;   // 96: 147 KB
+        const int mpmax = (EIGH_MAXN + 15) & ~15;   // 96: 74 KB
         if (hipFuncSetAttribute((const void*)purify_small_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * 2 * mpmax * mpmax)) != hipSuccess)
+                                (int)(sizeof(double) * mpmax * mpmax)) != hipSuccess)
             return pq_set_error("pq_purify_batched: cannot raise the kernel's LDS limit");
         attr = true;
     }
-    hipLaunchKernelGGL(purify_small_kernel, dim3(batch), dim3(256), lds, (hipStream_t)stream, M, nocc, m, tol,
+    hipLaunchKernelGGL(purify_small_kernel, dim3(batch), dim3(64 * PURIFY_W), lds, (hipStream_t)stream, M, nocc, m, tol,
                        max_steps, P, steps);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return pq_set_error((std::string("pq_purify_batched: ") + hipGetErrorString(e)).c_str());

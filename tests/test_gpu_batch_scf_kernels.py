@@ -118,3 +118,47 @@ def test_lift(gpu, m):
     t = torch.as_tensor(M.copy(), device="cuda")
     _call("pq_batch_lift", 3, m, t, torch.as_tensor(drop, device="cuda"))
     assert (np.abs(t.cpu().numpy() - ref) <= (m + 8) * U * (np.abs(M).sum(2).max((1,), keepdims=True) + 2)[:, :, None]).all()
+
+
+def _tc2(A, nocc, tol=1e-11, max_steps=200):
+    """The purification over the whole matrix: (P, steps)."""
+    d = np.diag(A)
+    rad = np.abs(A).sum(1) - np.abs(d)
+    lo, hi = (d - rad).min(), (d + rad).max()
+    X, last, k = (hi * np.eye(len(A)) - A) / (hi - lo), False, 0
+    while k < max_steps:
+        X2 = X @ X
+        t1, t2 = np.trace(X), np.trace(X2)
+        X = X2 if abs(t2 - nocc) < abs(2 * t1 - t2 - nocc) else 2 * X - X2
+        if last:
+            break
+        last = t1 - t2 < tol
+        k += 1
+    return 0.5 * (X + X.T), k + 1 if last else max_steps + 1
+
+
+@pytest.mark.parametrize("m,coupled", [(5, 0), (16, 15), (17, 16), (33, 17), (48, 48), (61, 7), (90, 65), (90, 90)])
+def test_projectors_with_uncoupled_rows(gpu, m, coupled):
+    """Trailing rows that couple to nothing, above the rest or among its
+    levels, against the same steps over the whole matrix.  The purified X is
+    idempotent to 1e-11 before the last squaring and the spectra have a gap of
+    1 at the Fermi level: 1e-10."""
+    import torch
+    from pychem_amd.engine import purify_batched
+    rng = np.random.default_rng(m + 100 * coupled)
+    A, nocc = np.zeros((4, m, m)), np.zeros(4, dtype=np.int64)
+    for b in range(4):
+        low = rng.integers(0, m + 1)
+        lam = np.concatenate([rng.uniform(-3, -0.5, low), rng.uniform(0.5, 3, m - low)])
+        rng.shuffle(lam)
+        Q = np.eye(m)
+        if coupled:
+            Q[:coupled, :coupled] = np.linalg.qr(rng.normal(size=(coupled, coupled)))[0]
+        A[b] = (Q * lam) @ Q.T
+        A[b] = 0.5 * (A[b] + A[b].T)
+        nocc[b] = low
+    P, steps = purify_batched(torch.as_tensor(A, device="cuda"), nocc)
+    for b in range(4):
+        ref, k = _tc2(A[b], nocc[b])
+        assert np.abs(P[b].cpu().numpy() - ref).max() < 1e-10
+        assert int(steps[b]) == k
