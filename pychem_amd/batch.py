@@ -31,21 +31,22 @@ class BatchEngine:
             raise _lib.HipError("no GPU visible: the HIP engine has no CPU fallback")
         self.mols = mols
         self.device = torch.device(device)
-        tabs = [m.shell_table() for m in mols]
-        for t in tabs:
-            if t["nao"] != t["ncart_total"]:
+        tabs = [m.shell_layout() for m in mols]
+        for m, t in zip(mols, tabs):
+            if int(m.NOrbitals) != t["ncart_total"]:
                 raise ValueError("batched path expects Cartesian-basis molecules (cartesian_l covering d)")
         l = np.concatenate([t["l"] for t in tabs]).astype(np.int32)
         nprim = np.concatenate([t["nprim"] for t in tabs]).astype(np.int32)
         prim_off = np.zeros(len(l), dtype=np.int32)
         prim_off[1:] = np.cumsum(nprim)[:-1]
-        center = np.concatenate([t["center"] for t in tabs]).astype(float)
         exps = np.concatenate([t["exps"] for t in tabs]).astype(float)
         cc = np.concatenate([t["cc"] for t in tabs]).astype(float)
         shell_mol = np.repeat(np.arange(len(tabs), dtype=np.int32), [t["nshell"] for t in tabs])
-        axyz = np.concatenate([t["atom_xyz"] for t in tabs]).astype(float)
-        az = np.concatenate([t["atom_z"] for t in tabs]).astype(float)
-        amol = np.repeat(np.arange(len(tabs), dtype=np.int32), [t["natom"] for t in tabs])
+        xyz = np.array([a.Coordinates for m in mols for a in m.Atoms], dtype=float).reshape(-1, 3)
+        center = np.repeat(xyz, np.concatenate([t["per_atom"] for t in tabs]), axis=0).reshape(-1)
+        axyz = xyz.reshape(-1)
+        az = np.array([a.NuclearCharge for m in mols for a in m.Atoms], dtype=float)
+        amol = np.repeat(np.arange(len(tabs), dtype=np.int32), [m.NAtom for m in mols])
         self._keep = (l, nprim, prim_off, center, exps, cc, shell_mol, axyz, az, amol)
         h = ctypes.c_void_p()
         L = _lib.lib()
@@ -149,20 +150,19 @@ class BatchEngine:
         check(_lib.lib().pq_jk(self.h, _ptr(self.Dj), _ptr(self.Dk), _ptr(self.J), _ptr(self.K), _stream()), "pq_jk")
 
 
-def _sad_padded(eng, mols, host=False):
-    """SAD densities [B, nmax, nmax] (device; numpy with host=True)."""
+def _sad_packed(eng, mols):
+    """SAD densities, packed (host): a quarter of the padded matrices' bytes
+    for 512 molecules of 7 to 61 functions."""
     from .guess import sad_density
-    B, nm = eng.nmol, eng.nmax
-    D = np.zeros((B, nm, nm))
+    D = np.empty(eng.mat_total)
     layouts = {}   # one SAD matrix per layout (basis, atom labels, Cartesian shells) of this batch
     for m, mol in enumerate(mols):
         key = (mol.Basis, tuple(a.Label for a in mol.Atoms), tuple(mol.CartesianL))
         d = layouts.get(key)
         if d is None:
-            d = layouts[key] = sad_density(mol)
-        n = d.shape[0]
-        D[m, :n, :n] = d
-    return D if host else torch.as_tensor(D).to(eng.device)
+            d = layouts[key] = np.asarray(sad_density(mol), dtype=float).reshape(-1)
+        D[eng.base[m]:eng.base[m] + d.size] = d
+    return D
 
 
 def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_graph=True, diis_size=8,
@@ -201,11 +201,11 @@ def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_grap
     # copies to the device then wait for that work
     nocc_h = np.array([m.NAlphaElectrons for m in mols])
     enuc_h = _nuclear_batch(eng)
-    D_h = _sad_padded(eng, mols, host=True) if guess == "SAD" else None
+    D_h = _sad_packed(eng, mols) if guess == "SAD" else None
     nocc = torch.as_tensor(nocc_h, device=dev).to(torch.int32)
     enuc = torch.as_tensor(enuc_h, dtype=torch.float64, device=dev)
     if guess == "SAD":
-        D = 0.5 * torch.as_tensor(D_h).to(dev)
+        D = 0.5 * eng.to_padded(torch.as_tensor(D_h).to(dev))
     else:
         D = _density(X, Hp, dropped, nocc)
     if tune is not None:
@@ -288,8 +288,9 @@ def rhf_batch(mols, conv=1e-8, maxiter=60, threshold=1e-8, guess="SAD", use_grap
                latency_s=latency, total_s=total, setup_s=t_setup, nmol=B, stats=eng.stats(),
                tuned=getattr(eng, "tuned", None))
     if return_density:
-        Dh = D.cpu().numpy()
-        out["densities"] = [Dh[m, :eng.n[m], :eng.n[m]].copy() for m in range(B)]
+        Dh = eng.to_packed(D).cpu().numpy()
+        out["densities"] = [Dh[eng.base[m]:eng.base[m] + int(eng.n[m]) ** 2].reshape(eng.n[m], eng.n[m]).copy()
+                            for m in range(B)]
     eng.close()
     return out
 

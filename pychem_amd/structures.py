@@ -284,11 +284,11 @@ class Molecule:
         return self._shell_pairs
 
     # ------------------------------------------------------------------ #
-    def shell_table(self):
-        """Flat per-shell arrays consumed by the HIP library and the oracle.
-        Everything but the coordinates depends only on the basis, the atoms'
-        labels in order and the Cartesian shells, and is built once per such
-        layout (molecules of a batch share a handful of layouts)."""
+    def shell_layout(self):
+        """The arrays of ``shell_table`` that do not hold coordinates: they
+        depend only on the basis, the atoms' labels in order and the Cartesian
+        shells, and are built once per such layout (molecules of a batch share
+        a handful of layouts).  Shared: not to be written to."""
         key = (self.Basis, tuple(a.Label for a in self.Atoms), tuple(self.CartesianL))
         lay = _SHELL_LAYOUTS.get(key)
         if lay is None:
@@ -309,6 +309,12 @@ class Molecule:
             lay = dict(nshell=ns, l=l, nprim=nprim, prim_off=prim_off, spher=spher, exps=exps, cc=cc,
                        ao_off=ao_off, nfun=nfun, cart_off=cart_off, ncart_total=int(nc.sum()), per_atom=per_atom)
             _SHELL_LAYOUTS[key] = lay
+        return lay
+
+    def shell_table(self):
+        """Flat per-shell arrays consumed by the HIP library and the oracle
+        (the caller's own copies)."""
+        lay = self.shell_layout()
         xyz = np.array([a.Coordinates for a in self.Atoms], dtype=float)
         center = np.ascontiguousarray(np.repeat(xyz, lay["per_atom"], axis=0).reshape(-1))
         out = {k: (v.copy() if isinstance(v, np.ndarray) else v) for k, v in lay.items() if k != "per_atom"}
