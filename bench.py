@@ -319,8 +319,8 @@ FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense FP32 matrix
 
 
 def mlp_measure(name, reps=10, batch=4096):
-    """The learned guess's networks on the matrix cores (pq_mlp_linear_fwd /
-    _bwd, v_mfma_f32_16x16x4f32): the inference over every atom-pair group of
+    """The learned guess's networks on the matrix cores (pq_mlp_forward /
+    _backward, v_mfma_f32_16x16x4f32): the inference over every atom-pair group of
     the workload (what a solve with the learned guess runs) and one training
     step (forward and backward) of the largest network on a batch, each timed
     with HIP events on the working stream.  Flops: 2 B sum(in x out) per

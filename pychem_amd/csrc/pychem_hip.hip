@@ -506,26 +506,36 @@ static int ensure_events(pq_basis* b)
     return 0;
 }
 
-// Per class: the call's span (set = 0: empty it; 1: add it to the sums; 2:
-// clear everything).
-__global__ void jk_clock_kernel(unsigned long long* clock, int set)
+// Per class (a block of one wave, a lane per slot): the call's span (set = 0:
+// empty it; 1: add it to the sums; 2: clear everything).  The sums lie behind
+// the slots.
+#define JK_CLOCK_SUMS (2 * JK_CLOCK_SLOTS * JK_CLOCK_CLASSES)
+static_assert(ERI_NCLASS <= JK_CLOCK_CLASSES && JK_CLOCK_SLOTS == 64, "one wave per class");
+__global__ void __launch_bounds__(64) jk_clock_kernel(unsigned long long* clock, int set)
 {
-    const int c = threadIdx.x;
-    if (c >= ERI_NCLASS) return;
-    unsigned long long* sum = clock + 2 * ERI_NCLASS;
-    if (set == 2) sum[2 * c] = sum[2 * c + 1] = 0;
-    if (set == 1 && clock[2 * c + 1] > clock[2 * c]) {
-        sum[2 * c] += clock[2 * c + 1] - clock[2 * c];
-        sum[2 * c + 1] += 1;
+    const int c = blockIdx.x;
+    unsigned long long* at = clock + jk_clock_at(threadIdx.x, c);
+    unsigned long long lo = at[0], hi = at[1];
+    at[0] = ~0ULL;
+    at[1] = 0;
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long l = __shfl_xor(lo, o, 64), h = __shfl_xor(hi, o, 64);
+        lo = l < lo ? l : lo;
+        hi = h > hi ? h : hi;
     }
-    clock[2 * c] = ~0ULL;
-    clock[2 * c + 1] = 0;
+    if (threadIdx.x) return;
+    unsigned long long* sum = clock + JK_CLOCK_SUMS + 2 * c;
+    if (set == 2) sum[0] = sum[1] = 0;
+    if (set == 1 && hi > lo) {
+        sum[0] += hi - lo;
+        sum[1] += 1;
+    }
 }
 
 static void jk_clock_set(pq_basis* b, int set, hipStream_t st)
 {
     if (b->timing && b->d_jkclock.p)
-        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, st, (unsigned long long*)b->d_jkclock.p, set);
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(ERI_NCLASS), dim3(64), 0, st, (unsigned long long*)b->d_jkclock.p, set);
 }
 
 extern "C" const char* pq_last_error(void) { return g_err.c_str(); }
@@ -1669,7 +1679,7 @@ extern "C" int pq_jk_class_times(pq_basis* b, double* sum_ms, long long* launche
         HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
         if (khz > 0) ms_per_tick = 1.0 / khz;
         HIPCHK(hipDeviceSynchronize());
-        HIPCHK(hipMemcpy(h, (unsigned long long*)b->d_jkclock.p + 2 * ERI_NCLASS, sizeof(h), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(h, (unsigned long long*)b->d_jkclock.p + JK_CLOCK_SUMS, sizeof(h), hipMemcpyDeviceToHost));
     }
     for (int c = 0; c < ERI_NCLASS; ++c) {
         if (sum_ms) sum_ms[c] = (double)h[2 * c] * ms_per_tick;
@@ -1677,7 +1687,7 @@ extern "C" int pq_jk_class_times(pq_basis* b, double* sum_ms, long long* launche
         if (nitems) nitems[c] = b->store64[c].nitems;
     }
     if (reset && b->d_jkclock.p) {
-        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(ERI_NCLASS), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
         HIPCHK(hipDeviceSynchronize());
     }
     return 0;
@@ -1690,8 +1700,8 @@ extern "C" int pq_set_timing(pq_basis* b, int on)
     if (!b->timing) return 0;
     if (ensure_events(b)) return -1;
     if (!b->d_jkclock.p) {
-        if (b->d_jkclock.ensure(sizeof(unsigned long long) * 4 * ERI_NCLASS)) return -1;
-        hipLaunchKernelGGL(jk_clock_kernel, dim3(1), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
+        if (b->d_jkclock.ensure(sizeof(unsigned long long) * (JK_CLOCK_SUMS + 2 * ERI_NCLASS))) return -1;
+        hipLaunchKernelGGL(jk_clock_kernel, dim3(ERI_NCLASS), dim3(64), 0, nullptr, (unsigned long long*)b->d_jkclock.p, 2);
         HIPCHK(hipDeviceSynchronize());
     }
     return 0;
