@@ -4,14 +4,23 @@
 // One workgroup per matrix, the matrix and the accumulated rotations in LDS.
 // Cyclic Jacobi in the round-robin (tournament) order: index 0 stays, the
 // others rotate one place per round, so each of the m - 1 rounds of a sweep
-// (m = n rounded up to even) rotates m / 2 disjoint pairs together.  Each
-// rotation zeroes its pair's off-diagonal element, with Rutishauser's
-// formula: theta = (a_qq - a_pp) / (2 a_pq), t = sign(theta) / (|theta| +
-// sqrt(theta^2 + 1)), c = 1 / sqrt(t^2 + 1), s = t c, and rows, then columns
-// of A and the columns of V are updated as A <- J^T A J, V <- V J.  Sweeps
-// stop when the off-diagonal sum of squares is below 1e-30 times the
-// diagonal's.  Eigenvalues are returned in ascending order with their
-// eigenvectors as columns.
+// rotates m / 2 disjoint pairs together (m: the last row that couples to
+// another, plus one, rounded up to even; the rows behind it, a small
+// molecule's padding, are eigenvectors as they stand).  Each rotation zeroes
+// its pair's off-diagonal element, with Rutishauser's formula: theta = (a_qq -
+// a_pp) / (2 a_pq), t = sign(theta) / (|theta| + sqrt(theta^2 + 1)), c = 1 /
+// sqrt(t^2 + 1), s = t c, and rows, then columns of A and the columns of V are
+// updated as A <- J^T A J, V <- V J: the 2 x 2 block of two pairs by one lane,
+// rows and columns in one pass, a half wave or a wave along one pair's row of
+// blocks.  Sweeps stop when the off-diagonal sum of squares is below 1e-30
+// times the diagonal's (of the coupled rows: a padding of 1e3 must not loosen
+// it).  Eigenvalues are returned in ascending order with
+// their eigenvectors as columns.
+//
+// Bound by the rounds' latency (two barriers and the chain of two divisions
+// and two square roots): 512 matrices of 61 rows, molecules of 7 to 61
+// functions, 1.44 ms (2.97 with the padding rotated too, separate passes over
+// rows and columns and a division per element).
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -34,39 +43,52 @@ __device__ __forceinline__ double eigh_block_sum(double v, double* red)
     return s;
 }
 
-__global__ void __launch_bounds__(256) eigh_jacobi_kernel(const double* __restrict__ A, int n,
-                                                          double* __restrict__ w, double* __restrict__ V)
+#define EIGH_W 8        // waves per matrix
+__global__ void __launch_bounds__(64 * EIGH_W) eigh_jacobi_kernel(const double* __restrict__ A, int n,
+                                                                  double* __restrict__ w, double* __restrict__ V)
 {
     extern __shared__ double sh[];
     double* a = sh;           // n x n, row-major
     double* v = sh + n * n;   // n x n, the rotations' product
     __shared__ double cs[EIGH_MAXN / 2 + 1], sn[EIGH_MAXN / 2 + 1];
     __shared__ int pp[EIGH_MAXN / 2 + 1], qq[EIGH_MAXN / 2 + 1];
-    __shared__ int perm[EIGH_MAXN];
-    __shared__ double red[16];
-    const int tid = threadIdx.x, nt = blockDim.x;
+    __shared__ int perm[EIGH_MAXN], s_me;
+    __shared__ double red[16], lam[EIGH_MAXN];
+    const int tid = threadIdx.x, nt = 64 * EIGH_W, wave = tid >> 6, lane = tid & 63;
     const size_t off = (size_t)blockIdx.x * n * n;
-    for (int i = tid; i < n * n; i += nt) {
-        a[i] = A[off + i];
-        v[i] = (i / n == i % n) ? 1.0 : 0.0;
-    }
+    if (tid == 0) s_me = 0;
     __syncthreads();
-    const int m = n + (n & 1);   // index n is a dummy when n is odd
+    int me = 0;
+    for (int i = tid; i < n * n; i += nt) {
+        const int r = i / n, c = i - r * n;
+        const double x = A[off + i];
+        a[i] = x;
+        v[i] = r == c ? 1.0 : 0.0;
+        if (r != c && x != 0.0) me = max(me, max(r, c) + 1);
+    }
+    if (me) atomicMax(&s_me, me);
+    __syncthreads();
+    me = s_me;
+    const int m = me + (me & 1);   // index me is a dummy when me is odd
     const int np = m / 2;
+    // a row of 2 x 2 blocks along a half wave, two rows a wave, up to 64 players
+    const int half = np <= 32 ? 32 : 64, pj = lane & (half - 1), pi0 = wave * (64 / half) + lane / half,
+              pis = EIGH_W * (64 / half);
     for (int sweep = 0; sweep < EIGH_MAX_SWEEPS; ++sweep) {
         double o = 0.0, d = 0.0;
-        for (int i = tid; i < n * n; i += nt) {
-            const int r = i / n, c = i % n;
-            if (r < c) o += a[i] * a[i];
-            else if (r == c) d += a[i] * a[i];
-        }
+        for (int r = wave; r < me; r += EIGH_W)
+            for (int c = r + 1 + lane; c < me; c += 64) o += a[r * n + c] * a[r * n + c];
+        for (int i = tid; i < me; i += nt) d += a[i * n + i] * a[i * n + i];
         o = eigh_block_sum(o, red);
         d = eigh_block_sum(d, red);
         if (o <= 1e-30 * d || o == 0.0) break;
         for (int round = 0; round < m - 1; ++round) {
             if (tid < np) {
                 // players at positions tid and m - 1 - tid of this round
-                auto player = [&](int k) { return k == 0 ? 0 : ((k - 1 + round) % (m - 1)) + 1; };
+                auto player = [&](int k) {
+                    const int x = k - 1 + round;   // < 2 (m - 1)
+                    return k == 0 ? 0 : (x >= m - 1 ? x - (m - 1) : x) + 1;
+                };
                 int p = player(tid), q = player(m - 1 - tid);
                 if (p > q) {
                     const int x = p;
@@ -74,7 +96,7 @@ __global__ void __launch_bounds__(256) eigh_jacobi_kernel(const double* __restri
                     q = x;
                 }
                 double c = 1.0, s = 0.0;
-                if (q < n) {
+                if (q < me) {
                     const double apq = a[p * n + q];
                     if (apq != 0.0) {
                         const double theta = (a[q * n + q] - a[p * n + p]) / (2.0 * apq);
@@ -84,51 +106,70 @@ __global__ void __launch_bounds__(256) eigh_jacobi_kernel(const double* __restri
                     }
                 }
                 pp[tid] = p;
-                qq[tid] = q < n ? q : p;   // a dummy pair rotates nothing
+                qq[tid] = q < me ? q : -1;   // a dummy pair rotates nothing
                 cs[tid] = c;
                 sn[tid] = s;
             }
             __syncthreads();
-            for (int idx = tid; idx < np * n; idx += nt) {   // rows p, q of A
-                const int j = idx / n, k = idx - j * n;
-                const int p = pp[j], q = qq[j];
-                if (p == q) continue;
-                const double c = cs[j], s = sn[j];
-                const double x = a[p * n + k], y = a[q * n + k];
-                a[p * n + k] = c * x - s * y;
-                a[q * n + k] = s * x + c * y;
+            if (pj < np) {   // rows of pair i, then columns of pair j
+                const int pc = pp[pj], qc = qq[pj];
+                const double cj = cs[pj], sj = sn[pj];
+                for (int i = pi0; i < np; i += pis) {
+                    const int pr = pp[i], qr = qq[i];
+                    const double ci = cs[i], si = sn[i];
+                    double* const x0 = a + pr * n;
+                    double* const x1 = a + max(qr, 0) * n;
+                    double a00 = x0[pc], a01 = qc >= 0 ? x0[qc] : 0.0;
+                    double a10 = 0.0, a11 = 0.0;
+                    if (qr >= 0) {
+                        a10 = x1[pc];
+                        a11 = qc >= 0 ? x1[qc] : 0.0;
+                        const double t0 = ci * a00 - si * a10, t1 = ci * a01 - si * a11;
+                        a10 = si * a00 + ci * a10;
+                        a11 = si * a01 + ci * a11;
+                        a00 = t0;
+                        a01 = t1;
+                    }
+                    if (qc >= 0) {
+                        const double t0 = cj * a00 - sj * a01, t1 = cj * a10 - sj * a11;
+                        a01 = sj * a00 + cj * a01;
+                        a11 = sj * a10 + cj * a11;
+                        a00 = t0;
+                        a10 = t1;
+                        x0[qc] = a01;
+                        if (qr >= 0) x1[qc] = a11;
+                    }
+                    x0[pc] = a00;
+                    if (qr >= 0) x1[pc] = a10;
+                }
             }
-            __syncthreads();
-            for (int idx = tid; idx < np * n; idx += nt) {   // columns p, q of A and V
-                const int j = idx / n, k = idx - j * n;
+            for (int j = wave; j < np; j += EIGH_W) {   // columns p, q of V
                 const int p = pp[j], q = qq[j];
-                if (p == q) continue;
+                if (q < 0) continue;
                 const double c = cs[j], s = sn[j];
-                const double x = a[k * n + p], y = a[k * n + q];
-                a[k * n + p] = c * x - s * y;
-                a[k * n + q] = s * x + c * y;
-                const double xv = v[k * n + p], yv = v[k * n + q];
-                v[k * n + p] = c * xv - s * yv;
-                v[k * n + q] = s * xv + c * yv;
+                for (int k = lane; k < me; k += 64) {
+                    const double xv = v[k * n + p], yv = v[k * n + q];
+                    v[k * n + p] = c * xv - s * yv;
+                    v[k * n + q] = s * xv + c * yv;
+                }
             }
             __syncthreads();
         }
     }
-    if (tid == 0) {   // ascending order of the eigenvalues (selection sort, n <= 90)
-        for (int i = 0; i < n; ++i) perm[i] = i;
-        for (int i = 0; i < n; ++i) {
-            int best = i;
-            for (int j = i + 1; j < n; ++j)
-                if (a[perm[j] * n + perm[j]] < a[perm[best] * n + perm[best]]) best = j;
-            const int x = perm[i];
-            perm[i] = perm[best];
-            perm[best] = x;
-        }
+    for (int i = tid; i < n; i += nt) {
+        lam[i] = a[i * n + i];
+        perm[i] = i;
     }
     __syncthreads();
-    for (int i = tid; i < n; i += nt) w[(size_t)blockIdx.x * n + i] = a[perm[i] * n + perm[i]];
+    for (int i = tid; i < n; i += nt) {   // ascending order, equal ones as they come
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += lam[j] < lam[i] || (lam[j] == lam[i] && j < i);
+        perm[rank] = i;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += nt) w[(size_t)blockIdx.x * n + i] = lam[perm[i]];
     for (int i = tid; i < n * n; i += nt) {
-        const int r = i / n, c = i % n;
+        const int r = i / n, c = i - r * n;
         V[off + i] = v[r * n + perm[c]];
     }
 }
@@ -149,7 +190,7 @@ extern "C" int pq_eigh_batched(const double* A, int batch, int n, double* w, dou
             return pq_set_error("pq_eigh_batched: cannot raise the kernel's LDS limit");
         attr = true;
     }
-    hipLaunchKernelGGL(eigh_jacobi_kernel, dim3(batch), dim3(256), lds, (hipStream_t)stream, A, n, w, V);
+    hipLaunchKernelGGL(eigh_jacobi_kernel, dim3(batch), dim3(64 * EIGH_W), lds, (hipStream_t)stream, A, n, w, V);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return pq_set_error((std::string("pq_eigh_batched: ") + hipGetErrorString(e)).c_str());
     return 0;

@@ -162,3 +162,25 @@ def test_projectors_with_uncoupled_rows(gpu, m, coupled):
         ref, k = _tc2(A[b], nocc[b])
         assert np.abs(P[b].cpu().numpy() - ref).max() < 1e-10
         assert int(steps[b]) == k
+
+
+@pytest.mark.parametrize("n,coupled", [(1, 0), (5, 0), (16, 2), (17, 16), (61, 7), (64, 64), (65, 63), (90, 89)])
+def test_eigenpairs_with_uncoupled_rows(gpu, n, coupled):
+    """Trailing rows that couple to nothing, repeated levels among them.  The
+    sweeps stop at 1e-15 of the diagonal; each of some 10 sweeps of n rounds
+    rounds an element twice: 20 n u of the norm at most, 1e-12 at n = 90."""
+    import torch
+    from pychem_amd.engine import eigh_batched
+    rng = np.random.default_rng(7 * n + coupled)
+    A = np.zeros((3, n, n))
+    for b in range(3):
+        A[b] = np.diag(rng.integers(-3, 4, n).astype(float))
+        B = rng.normal(size=(coupled, coupled))
+        A[b, :coupled, :coupled] = B + B.T
+    w, V = (x.cpu().numpy() for x in eigh_batched(torch.as_tensor(A, device="cuda")))
+    ref = np.linalg.eigvalsh(A)
+    scale = max(1.0, np.abs(ref).max())
+    assert np.abs(w - ref).max() <= 1e-12 * scale
+    for b in range(3):
+        assert np.abs(A[b] @ V[b] - V[b] * w[b]).max() <= 1e-12 * scale
+        assert np.abs(V[b].T @ V[b] - np.eye(n)).max() <= 1e-12
