@@ -457,8 +457,8 @@ struct pq_basis {
     hipGraphExec_t graph_exec = nullptr;
     // Class launches fan out over side streams (default priority); with the
     // caller's stream, four streams fill the process's four hardware queues.
-    // J/K: jk_nstreams streams, the caller's one of them (C20H42: 1.24 ms on
-    // one, 1.21 on four).  Schwarz and ERI passes: eri_nstreams side
+    // J/K: jk_nstreams streams, the caller's one of them (C20H42: 1.18 ms on
+    // one, 1.12 on four).  Schwarz and ERI passes: eri_nstreams side
     // streams beside the caller's, which runs the classes that use scratch.
     int jk_nstreams = 4;
     int eri_nstreams = 3;
